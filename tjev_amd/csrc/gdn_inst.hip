@@ -188,8 +188,7 @@ hipError_t run(const GdnArgs& A, hipStream_t st, int backward, const Timer* tm) 
       }
     } else if (A.ny) GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO, true>), persist, dim3(C * 4));
     else GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO>), persist, dim3(C * 4));
-    if (A.final_state) GDN_LAUNCH(K_FINAL_STATE, (k_final_state<C, D>), dim3(A.B * A.H * (D / DVT)), dim3(256));
-    if (A.conv_state && A.taps > 1) GDN_LAUNCH(K_FINAL_STATE, (k_conv_state<TIO>), dim3(A.B), dim3(256));
+    if (const unsigned tail = tail_blocks<D, TIO>(A)) GDN_LAUNCH(K_FINAL_STATE, (k_tail<C, D, TIO>), dim3(tail), dim3(256));
   } else {
     const int wouts = A.d_conv_w ? A.taps * A.W : 0;  // one workgroup per head, then the conv weights
     if (A.taps <= 4) GDN_LAUNCH(K_PREP_BWD, (k_prep<C, D, TIO, TG, 3>), prep, dim3(256));
@@ -256,7 +255,7 @@ hipError_t run_v2(const GdnArgs& A, hipStream_t st, int backward, const Timer* t
     if constexpr (C == 128 && D == 128) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_split<PI, PS>), tiles, dim3(512));
     else GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd<C, D, DVT, PI, PS>), tiles, dim3(NS));
     GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO>), persist, dim3(C * 4));
-    if (A.final_state) GDN_LAUNCH(K_FINAL_STATE, (k_final_state<C, D>), dim3(A.B * A.H * (D / DVT)), dim3(256));
+    if (const unsigned tail = tail_blocks<D, TIO>(A)) GDN_LAUNCH(K_FINAL_STATE, (k_tail<C, D, TIO>), dim3(tail), dim3(256));
   } else {
     GDN_LAUNCH(K_PREP_BWD, (k_prep_v2<C, D, TIO, TQK, TG>), ends, dim3(256));
     if (A.res == 0) {

@@ -29,7 +29,7 @@ namespace gdn {
 // (pallas_tpu_mega.py:425-426, _state_dtypes). Every reader of S in those modes feeds it to a
 // one-pass bf16 product, which rounds it to bf16 anyway, except the carry's gradient
 // <G_after, S_before> (the reference reads its bf16 S there too) and the final state, which
-// k_final_state builds from an fp32 copy of the last chunk's S (GdnArgs::s_last).
+// k_tail builds from an fp32 copy of the last chunk's S (GdnArgs::s_last).
 template <int PS>
 using StateT = std::conditional_t<PS == P_BF16, uint16_t, float>;
 template <int PS>
@@ -1979,79 +1979,132 @@ __global__ __launch_bounds__(C * 4) void k_out(GdnArgs A) {
   }
 }
 
-// ---------------------------------------------------------------- k_final_state
-// grid B*H*(D/DT), 256 threads: the recurrent state after token T-1 of each row, for a decode
-// step that continues it (xla.py:141-167 run to the last token). It is the scan's update of
-// the last chunk with T-1 as that chunk's last token (the chunk step, pallas_tpu_v2.py:254-269,
-// truncated there): S = carry' S_before + sum over the chunk's tokens t <= T-1 of token T-1's
-// segment of e^(gamma_{T-1} - gamma_t) k_t v_new_t^T, carry' = e^(gamma_{T-1}) when that
-// segment began before the chunk. The rows of v_new up to T-1 do not depend on later rows.
-template <int C, int D>
-__global__ __launch_bounds__(256) void k_final_state(GdnArgs A) {
-  constexpr int DT = D < 32 ? D : 32;
-  constexpr int NTL = D / DT;
-  constexpr int RG = 256 / DT;              // row groups of a tile
-  constexpr int RPT = (D + RG - 1) / RG;    // rows per thread
-  __shared__ float sk[C * D];
-  __shared__ float sv[C * DT];
-  __shared__ float sw[C];
-  GDN_POISON_LDS(sk, sv, sw);
-  const int tile = blockIdx.x % NTL, bh = blockIdx.x / NTL, h = bh % A.H, b = bh / A.H, hk = h / A.ratio;
-  const int last = A.T - 1, nl = last / C, t0 = nl * C, cnt = last - t0 + 1;
+// ---------------------------------------------------------------- k_tail
+// The decode state a prefill leaves, in one launch of 256-thread workgroups: the recurrent state
+// after token T-1 of each row (the first tail_blocks() workgroups, when final_state is given) and
+// the conv history (the rest, when conv_state is given).
+//
+// The recurrent state (xla.py:141-167 run to the last token) is the scan's update of the last
+// chunk with T-1 as that chunk's last token (the chunk step, pallas_tpu_v2.py:254-269, truncated
+// there): S = carry' S_before + sum over the chunk's tokens t <= T-1 of token T-1's segment of
+// e^(gamma_{T-1} - gamma_t) k_t v_new_t^T, carry' = e^(gamma_{T-1}) when that segment began before
+// the chunk. The rows of v_new up to T-1 do not depend on later rows. Whatever the precision it
+// is an fp32 product, on the fp32 MFMA.
+//
+// A workgroup takes TailTile::R state rows by TailTile::T columns: 128 of them at 16 heads of
+// 128, and one round trip to memory (48 KB per workgroup, every load issued first) with 64 MFMAs
+// per wave behind it is what bounds it. The conv history is copied in 16-byte pieces, one per
+// thread. Measured (event times) against a VALU sum over tokens and one history workgroup per
+// row, which read a few bytes per thread and round trip: 66 -> 8 us at one row of 333 tokens (16
+// heads), 193 -> 12 us at one of 8192 (32 heads), 135 -> 14 us at four of 1500 (16 heads).
+template <int D>
+struct TailTile {
+  static constexpr int R = D < 64 ? D : 64, T = D < 32 ? D : 32;
+  static constexpr int PER_HEAD = (D / R) * (D / T);
+};
+
+template <int C, int D, class TIO>
+__global__ __launch_bounds__(256) void k_tail(GdnArgs A) {
+  constexpr int R = TailTile<D>::R, T = TailTile<D>::T;
+  // row strides of 16 words modulo the 64 banks: the four token rows that one MFMA operand read
+  // spans fall in distinct banks
+  constexpr int LK = R + 16, LV = T + 16;
+  __shared__ __align__(16) float sk[C * LK];
+  __shared__ __align__(16) float sv[C * LV];
+  GDN_POISON_LDS(sk, sv);
+  const int tid = threadIdx.x, last = A.T - 1;
+  const int nstate = A.final_state ? A.B * A.H * TailTile<D>::PER_HEAD : 0;
+  if ((int)blockIdx.x >= nstate) {
+    // the raw rows T-K+1 .. T-1 of each row (oldest first, [B, K-1, W]), zero outside token T-1's
+    // segment or before the row's start (there: the given history, if any): the conv history a
+    // decode step continuing that segment reads (the tap masks of causal_conv1d.py:10-17)
+    constexpr int E = 16 / sizeof(TIO);
+    const int k1 = A.taps - 1, wu = A.W / E, units = k1 * wu;  // 16-byte pieces per row
+    const int per = (units + 255) / 256, cb = (int)blockIdx.x - nstate, b = cb / per;
+    const int u = (cb - b * per) * 256 + tid;
+    if (u >= units) return;
+    const int r = u / wu, c = (u - r * wu) * E, t = last - k1 + 1 + r;
+    const int32_t* sg = A.seg + (size_t)b * A.T;
+    const TIO* hist = reinterpret_cast<const TIO*>(A.init_conv);
+    const bool keep = sg[t >= 0 ? t : 0] == sg[last] && (t >= 0 || hist);
+    uint4 v = make_uint4(0u, 0u, 0u, 0u);
+    if (keep) v = *reinterpret_cast<const uint4*>(halo_row<TIO>(A, reinterpret_cast<const TIO*>(A.qkv), b, t, c));
+    TIO* dst = reinterpret_cast<TIO*>(A.conv_state) + ((size_t)b * k1 + r) * A.W + c;
+    if (reinterpret_cast<uintptr_t>(A.conv_state) % 16 == 0) {
+      *reinterpret_cast<uint4*>(dst) = v;
+    } else {  // an unaligned output is taken as it is
+      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        if constexpr (sizeof(TIO) == 2) dst[e] = (TIO)(w[e / 2] >> (16 * (e % 2)));
+        else dst[e] = __uint_as_float(w[e]);
+      }
+    }
+    return;
+  }
+  const int bh = blockIdx.x / TailTile<D>::PER_HEAD, q = blockIdx.x % TailTile<D>::PER_HEAD;
+  const int i0 = (q / (D / T)) * R, j0 = (q % (D / T)) * T;
+  const int h = bh % A.H, b = bh / A.H, hk = h / A.ratio;
+  const int nl = last / C, t0 = nl * C, cnt = last - t0 + 1;
   const size_t tb = (size_t)b * A.Tp, th = (size_t)bh * A.Tp;
-  const float* kg = A.kn + ((size_t)(b * A.Hk + hk) * A.Tp + t0) * D;
-  const float* vg = A.vnew + (th + t0) * D + tile * DT;
-  for (int idx = threadIdx.x; idx < cnt * D; idx += 256) sk[idx] = kg[idx];
-  for (int idx = threadIdx.x; idx < cnt * DT; idx += 256) sv[idx] = vg[(size_t)(idx / DT) * D + idx % DT];
+  const float* kg = A.kn + ((size_t)(b * A.Hk + hk) * A.Tp + t0) * D + i0;
+  const float* vg = A.vnew + (th + t0) * D + j0;
+  Regs<C, R, 256> kr;
+  Regs<C, T, 256> vr;
+  kr.fetch(kg, D);
+  vr.fetch(vg, D);
   const int sl = A.segp[tb + last];
   const float gl = A.gam[th + last], ll = A.gaml[th + last];
-  for (int t = threadIdx.x; t < cnt; t += 256)
-    sw[t] = A.segp[tb + t0 + t] == sl ? expf((gl - A.gam[th + t0 + t]) + (ll - A.gaml[th + t0 + t])) : 0.f;
+  float wt[Regs<C, T, 256>::IT];  // the weight of the token row each slot of vr holds
+#pragma unroll
+  for (int it = 0; it < Regs<C, T, 256>::IT; ++it) {
+    const int r = min((tid + it * 256) / (T / 4), C - 1);
+    wt[it] = A.segp[tb + t0 + r] == sl ? expf((gl - A.gam[th + t0 + r]) + (ll - A.gaml[th + t0 + r])) : 0.f;
+  }
   const int before = nl > 0 ? A.segp[tb + t0 - 1] : (A.init_state ? A.segp[tb] : -2);
   const float carry = sl == before ? expf(gl + ll) : 0.f;
-  __syncthreads();
-  const int j = threadIdx.x % DT, rg = threadIdx.x / DT;
+  const int w = wave(), l = lane();
+  const bool on = 16 * w < R;
   const float* S = (A.s_last ? A.s_last + (size_t)bh * D * D
-                              : static_cast<const float*>(A.states) + ((size_t)bh * A.N + nl) * D * D) + tile * DT + j;
-  float acc[RPT];
+                              : static_cast<const float*>(A.states) + ((size_t)bh * A.N + nl) * D * D) +
+                   (size_t)i0 * D + j0;
+  f32x4 acc[T / 16];
 #pragma unroll
-  for (int r = 0; r < RPT; ++r) {
-    const int i = rg * RPT + r;
-    acc[r] = i < D ? carry * S[(size_t)i * D] : 0.f;
-  }
-  for (int t = 0; t < cnt; ++t) {
-    const float wv = sw[t] * sv[t * DT + j];
+  for (int t = 0; t < T / 16; ++t)
 #pragma unroll
-    for (int r = 0; r < RPT; ++r) {
-      const int i = rg * RPT + r;
-      if (i < D) acc[r] += sk[t * D + i] * wv;
-    }
-  }
-  float* dst = A.final_state + (size_t)bh * D * D + tile * DT + j;
+    for (int rr = 0; rr < 4; ++rr)
+      acc[t][rr] = on ? carry * S[(size_t)(16 * w + acc_row(rr)) * D + 16 * t + acc_col()] : 0.f;
+  kr.put_lds(sk, LK);
 #pragma unroll
-  for (int r = 0; r < RPT; ++r) {
-    const int i = rg * RPT + r;
-    if (i < D) dst[(size_t)i * D] = acc[r];
+  for (int it = 0; it < Regs<C, T, 256>::IT; ++it) {
+    if (!Regs<C, T, 256>::live(it)) continue;
+    const int idx = tid + it * 256, r = idx / (T / 4), c = 4 * (idx % (T / 4));
+    const float f = wt[it];
+    *reinterpret_cast<float4*>(sv + r * LV + c) =  // the rows past T-1 do not count, whatever they hold
+        r < cnt ? make_float4(vr.v[it].x * f, vr.v[it].y * f, vr.v[it].z * f, vr.v[it].w * f) : make_float4(0.f, 0.f, 0.f, 0.f);
   }
+  __syncthreads();
+  if (!on) return;
+  const float* ak = sk + (l >> 4) * LK + 16 * w + (l & 15);
+  const float* bv = sv + (l >> 4) * LV + (l & 15);
+  for (int s = 0; s < (cnt + 3) / 4; ++s) {
+    const float a = ak[4 * s * LK];
+#pragma unroll
+    for (int t = 0; t < T / 16; ++t)
+      acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bv[4 * s * LV + 16 * t], acc[t], 0, 0, 0);
+  }
+  float* dst = A.final_state + (size_t)bh * D * D + (size_t)i0 * D + j0;
+#pragma unroll
+  for (int t = 0; t < T / 16; ++t)
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) dst[(size_t)(16 * w + acc_row(rr)) * D + 16 * t + acc_col()] = acc[t][rr];
 }
 
-// ---------------------------------------------------------------- k_conv_state
-// grid B, 256 threads: the raw rows T-K+1 .. T-1 of each row (oldest first, [B, K-1, W]), zero
-// outside token T-1's segment or before the row's start (there: the given history, if any): the conv history a decode step
-// continuing that segment reads (the tap masks of causal_conv1d.py:10-17).
-template <class TIO>
-__global__ __launch_bounds__(256) void k_conv_state(GdnArgs A) {
-  const int b = blockIdx.x, k1 = A.taps - 1, last = A.T - 1;
-  const TIO* x = reinterpret_cast<const TIO*>(A.qkv);
-  TIO* dst = reinterpret_cast<TIO*>(A.conv_state) + (size_t)b * k1 * A.W;
-  const int sl = A.seg[(size_t)b * A.T + last];
-  const TIO* hist = reinterpret_cast<const TIO*>(A.init_conv);
-  for (long idx = threadIdx.x; idx < (long)k1 * A.W; idx += 256) {  // k1 W can pass 2^31 (W < 2^30)
-    const int r = (int)(idx / A.W), c = (int)(idx % A.W), t = last - k1 + 1 + r;
-    // rows before the row: the history of a continued sequence (token 0's segment)
-    const bool keep = A.seg[(size_t)b * A.T + (t >= 0 ? t : 0)] == sl && (t >= 0 || hist);
-    dst[idx] = !keep ? TIO(0) : t >= 0 ? x[((size_t)b * A.T + t) * A.W + c] : hist[((size_t)b * k1 + k1 + t) * A.W + c];
-  }
+// workgroups of k_tail
+template <int D, class TIO>
+inline unsigned tail_blocks(const GdnArgs& A) {
+  const long pieces = A.conv_state && A.taps > 1 ? (long)(A.taps - 1) * A.W / (16 / (long)sizeof(TIO)) : 0;
+  return (unsigned)((A.final_state ? (long)A.B * A.H * TailTile<D>::PER_HEAD : 0) + A.B * ((pieces + 255) / 256));
 }
 
 // ---------------------------------------------------------------- k_bwd_local
