@@ -87,6 +87,29 @@ __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float(((uin
 // (gfx950's v_cvt_pk_bf16_f32: round to nearest even, NaN stays NaN)
 __device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
+// two values as bf16 (round to nearest even) in one 32-bit word, the first in the low half. As a
+// conversion of a two-element vector it is one v_cvt_pk_bf16_f32; converted one by one and
+// packed it is two of them, a shift and an or (ROCm 7.2). The kernels that stage operands are
+// bound by such instructions beside their loads; measured at the 0.8B layer shape (4 rows of 4096 tokens, 16
+// heads): k_chunk forward 203 -> 191 us, backward 200 -> 188 us, k_out 211 -> 205 us, k_bwd_local 177 ->
+// 172 us, k_bwd_grads (its staging alone) 341 -> 333 us.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  const f32x2 v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+// the bf16x3 split of two values: hi = bf16(v), lo = bf16(v - hi) (v - hi is exact in fp32)
+struct Split2 {
+  uint32_t hi, lo;
+};
+__device__ __forceinline__ Split2 split2(float a, float b) {
+  Split2 s;
+  s.hi = pack2(a, b);
+  s.lo = pack2(a - __uint_as_float(s.hi << 16), b - __uint_as_float(s.hi & 0xffff0000u));
+  return s;
+}
+
 // A single fp32 store into LDS that the backend may not pair with its neighbours. ROCm 7.2's
 // SI load/store optimizer can merge two such stores into one ds_write2_b32 with a wrongly
 // scaled first offset (seen for 272/336-byte offsets: emitted as 17/84 dwords); the empty asm
@@ -107,8 +130,7 @@ __device__ __forceinline__ void st4_io(float* p, const float (&v)[4]) {
   *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
 }
 __device__ __forceinline__ void st4_io(uint16_t* p, const float (&v)[4]) {
-  *reinterpret_cast<uint2*>(p) = make_uint2((uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
-                                            (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16));
+  *reinterpret_cast<uint2*>(p) = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
 }
 
 // 8 consecutive elements (16-byte aligned for bf16, 32-byte for fp32) as floats
@@ -134,10 +156,8 @@ __device__ __forceinline__ void st8_io(float* p, const float (&v)[8]) {
   reinterpret_cast<float4*>(p)[1] = make_float4(v[4], v[5], v[6], v[7]);
 }
 __device__ __forceinline__ void st8_io(uint16_t* p, const float (&v)[8]) {
-  uint32_t w[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) w[e] = (uint32_t)f2bf(v[2 * e]) | ((uint32_t)f2bf(v[2 * e + 1]) << 16);
-  *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
+  *reinterpret_cast<uint4*>(p) =
+      make_uint4(pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7]));
 }
 // Nontemporal forms for the step's final outputs, which no later kernel of the step reads:
 // they are not kept in the caches the next kernels' inputs go through
@@ -258,19 +278,31 @@ template <> struct Frag<P_F32> { float v[8]; };
 template <> struct Frag<P_BF16> { bf16x8 hi; };
 template <> struct Frag<P_BF16X3> { bf16x8 hi, lo; };
 
+// A fragment from eight fp32 values, by pairs (split2) unless GDN_FRAG_PAIRS is 0 (gdn_inst.hip
+// sets it for a kernel that runs out of registers with them); the same values either way.
+#ifndef GDN_FRAG_PAIRS
+#define GDN_FRAG_PAIRS 1
+#endif
 template <int P>
 __device__ __forceinline__ Frag<P> make_frag(const float (&x)[8]) {
   Frag<P> f;
   if constexpr (P == P_F32) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) f.v[e] = x[e];
-  } else {
+  } else if constexpr (!GDN_FRAG_PAIRS) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) f.hi[e] = (__bf16)x[e];
     if constexpr (P == P_BF16X3) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) f.lo[e] = (__bf16)(x[e] - (float)f.hi[e]);
     }
+  } else if constexpr (P == P_BF16) {
+    f.hi = __builtin_bit_cast(
+        bf16x8, make_uint4(pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7])));
+  } else {
+    const Split2 a = split2(x[0], x[1]), b = split2(x[2], x[3]), c = split2(x[4], x[5]), d = split2(x[6], x[7]);
+    f.hi = __builtin_bit_cast(bf16x8, make_uint4(a.hi, b.hi, c.hi, d.hi));
+    f.lo = __builtin_bit_cast(bf16x8, make_uint4(a.lo, b.lo, c.lo, d.lo));
   }
   return f;
 }
@@ -358,13 +390,6 @@ template <class V> __device__ __forceinline__ ScaleKF<V> scale_k(V v, const floa
 
 
 // ---------------------------------------------------------------- pre-converted LDS operands
-// two values as bf16 (round to nearest even) in one 32-bit word, the first in the low half
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-  return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)a) | ((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)b) << 16);
-}
-// v - bf16(v): the part a bf16 pass drops (exact in fp32)
-__device__ __forceinline__ float lo_part(float v) { return v - (float)(__bf16)v; }
-
 // Op<P>: an operand tile in LDS, converted once when it is staged. Element (r, k) sits at
 // r*ld + k with the contraction index k contiguous (r: the M index of an A operand, the N index
 // of a B operand), so a fragment is one 16-byte read per plane. P_F32 keeps fp32; P_BF16 one bf16
@@ -436,24 +461,23 @@ struct Op<P_BF16X3> {
     lo[r * ld + k] = __builtin_bit_cast(uint16_t, (__bf16)(v - (float)h));
   }
   __device__ __forceinline__ void put2(int r, int k, float v0, float v1) const {
-    *reinterpret_cast<uint32_t*>(hi + r * ld + k) = pack2(v0, v1);
-    *reinterpret_cast<uint32_t*>(lo + r * ld + k) = pack2(lo_part(v0), lo_part(v1));
+    const Split2 s = split2(v0, v1);
+    *reinterpret_cast<uint32_t*>(hi + r * ld + k) = s.hi;
+    *reinterpret_cast<uint32_t*>(lo + r * ld + k) = s.lo;
   }
   // bf16-exact values: the high plane only (the tile then feeds P_X3_BEXACT products)
   __device__ __forceinline__ void put2_hi(int r, int k, float v0, float v1) const {
     *reinterpret_cast<uint32_t*>(hi + r * ld + k) = pack2(v0, v1);
   }
   __device__ __forceinline__ void put4(int r, int k, float v0, float v1, float v2, float v3) const {
-    *reinterpret_cast<uint2*>(hi + r * ld + k) = make_uint2(pack2(v0, v1), pack2(v2, v3));
-    *reinterpret_cast<uint2*>(lo + r * ld + k) =
-        make_uint2(pack2(lo_part(v0), lo_part(v1)), pack2(lo_part(v2), lo_part(v3)));
+    const Split2 a = split2(v0, v1), b = split2(v2, v3);
+    *reinterpret_cast<uint2*>(hi + r * ld + k) = make_uint2(a.hi, b.hi);
+    *reinterpret_cast<uint2*>(lo + r * ld + k) = make_uint2(a.lo, b.lo);
   }
   __device__ __forceinline__ void put8(int r, int k, const float (&v)[8]) const {
-    *reinterpret_cast<uint4*>(hi + r * ld + k) =
-        make_uint4(pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7]));
-    *reinterpret_cast<uint4*>(lo + r * ld + k) =
-        make_uint4(pack2(lo_part(v[0]), lo_part(v[1])), pack2(lo_part(v[2]), lo_part(v[3])),
-                   pack2(lo_part(v[4]), lo_part(v[5])), pack2(lo_part(v[6]), lo_part(v[7])));
+    const Split2 a = split2(v[0], v[1]), b = split2(v[2], v[3]), c = split2(v[4], v[5]), d = split2(v[6], v[7]);
+    *reinterpret_cast<uint4*>(hi + r * ld + k) = make_uint4(a.hi, b.hi, c.hi, d.hi);
+    *reinterpret_cast<uint4*>(lo + r * ld + k) = make_uint4(a.lo, b.lo, c.lo, d.lo);
   }
   template <int Q>
   __device__ __forceinline__ Frag<Q> frag(int r, int k) const {
@@ -464,6 +488,13 @@ struct Op<P_BF16X3> {
     return f;
   }
 };
+
+// A 128 x 128 operand as bf16 planes of rows of 16 units of 16 bytes, unit u of row r at u ^ swz(r):
+// 16-byte reads of one unit from 8 consecutive rows and transposing reads of two adjacent units
+// from 4 consecutive rows both fall in distinct banks.
+__device__ __forceinline__ int swz(int r) { return ((r & 3) << 1) | ((r >> 2) & 1); }
+// element offset of unit u of row r in such a plane
+__device__ __forceinline__ int swz_at(int r, int u) { return r * 128 + ((u ^ swz(r)) << 3); }
 
 // LDS bytes and carving of an R x K operand tile (16 bytes of padding per row)
 template <int P, int R, int K>

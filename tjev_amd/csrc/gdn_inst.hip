@@ -14,6 +14,11 @@
 #if GDN_PART == 2 || GDN_PART == 3 || GDN_PART == 4
 #define GDN_LANE_OFF32 1
 #endif
+// fragments converted value by value in k_bwd_grads: by pairs it spills 27 VGPRs instead of 11
+// (bf16 I/O at C = D = 128: 360 against 333 us)
+#if GDN_PART == 5
+#define GDN_FRAG_PAIRS 0
+#endif
 #include "gdn_kernels.h"
 #include "gdn_launch.h"
 #include "gdn_v2.h"

@@ -55,7 +55,7 @@ __device__ __forceinline__ void st8(float* p, const float (&v)[8]) {
 __device__ __forceinline__ void st8(uint16_t* p, const float (&v)[8]) {
   uint32_t w[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) w[e] = (uint32_t)f2bf(v[2 * e]) | ((uint32_t)f2bf(v[2 * e + 1]) << 16);
+  for (int e = 0; e < 4; ++e) w[e] = pack2(v[2 * e], v[2 * e + 1]);
   *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
