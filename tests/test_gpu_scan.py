@@ -1,0 +1,48 @@
+"""The forward scan at C = D = 128 (four compute waves in the bf16 modes): one chunk, a chunk's edge
+and several chunks, states that start given or reset inside, before and after a chunk, rows that
+are split into ranges at those resets, and grouped heads, in every precision. Outputs and final
+state against the oracle's fp64 token recurrence: 1e-5 at "highest", 1e-4 at "high" (three bf16
+passes drop terms of 2^-16 of each product's operands; the chunk's products compound a few of
+them), 3e-2 where the state path is one bf16 pass (2^-8, the reference's bar for those modes)."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from gdn_cases import rel
+
+pytestmark = pytest.mark.gpu
+
+TOL = {"highest": 1e-5, "high": 1e-4, "mixed": 3e-2, "bf16": 3e-2}
+
+
+@pytest.mark.parametrize("precision", list(TOL))
+@pytest.mark.parametrize("length,cuts,fresh", [(1, None, True), (128, None, False), (129, [128], True), (300, [127], False),
+                                               (700, [64, 128, 256, 500], True), (640, None, False)])
+def test_scan_fwd_matches_the_recurrence(precision, length, cuts, fresh):
+    from oracle.gdn_oracle import recurrent_gated_delta_rule
+    from tjev_amd.testing import cut_segments
+    from tjev_amd.v2 import chunk_gated_delta_rule_v2
+
+    gen = torch.Generator().manual_seed(length)
+    b, hk, h, d = 2, 1, 2, 128
+    nrm = torch.nn.functional.normalize
+    q = nrm(torch.randn(b, length, hk, d, generator=gen), dim=-1) * d ** -0.5
+    k = nrm(torch.randn(b, length, hk, d, generator=gen), dim=-1)
+    v = torch.randn(b, length, h, d, generator=gen)
+    g = -torch.rand(b, length, h, generator=gen) * 0.1
+    beta = torch.rand(b, length, h, generator=gen)
+    s0 = None if fresh else torch.randn(b, h, d, d, generator=gen) * 0.1
+    seg = torch.ones(b, length, dtype=torch.int32)
+    if cuts:
+        seg[1] = torch.from_numpy(cut_segments(length, cuts))
+    print(f"scan {precision} T={length} cuts={cuts} fresh={fresh}", flush=True)
+    out, state = chunk_gated_delta_rule_v2(*(x.cuda() for x in (q, k, v, g, beta, seg)), chunk=128, precision=precision,
+                                           initial_state=None if s0 is None else s0.cuda(), output_final_state=True)
+    torch.cuda.synchronize()
+    rep = [x.double().repeat_interleave(h // hk, 2) for x in (q, k)]
+    want, ws = recurrent_gated_delta_rule(*rep, v.double(), g.double(), beta.double(), seg,
+                                          *([] if s0 is None else [s0.double()]))
+    assert rel(out.cpu(), want) <= TOL[precision], rel(out.cpu(), want)
+    assert rel(state.cpu(), ws) <= TOL[precision], rel(state.cpu(), ws)

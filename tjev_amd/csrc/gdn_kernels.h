@@ -1345,6 +1345,9 @@ __device__ __forceinline__ int part_start(const GdnArgs& A, int b, int q, int* r
     int best = A.N;
     for (int i = 0; i < NT / 64; ++i) best = min(best, red[i]);
     __syncthreads();
+    // the same in every thread: a scalar, so that the scan's chunk index and the addresses and
+    // branches on it are scalar too (read back from LDS it is a per-lane value to the compiler)
+    best = __builtin_amdgcn_readfirstlane(best);
     if (best < A.N) return best;
   }
   return A.N;
@@ -1485,7 +1488,7 @@ __global__ __launch_bounds__((C > D ? C : D) * 4) void k_scan_fwd(GdnArgs A) {
 }
 
 // ---------------------------------------------------------------- k_scan_fwd_split
-// The forward scan at C = D = 128 with its two products chained in registers. Two compute
+// The forward scan at C = D = 128 in the fp32 mode (the bf16 modes: k_scan_fwd_quad), with its two products chained in registers. Two compute
 // waves each own 16 value columns of the 32-column Dv tile: S[:, cols] (Dk x 16, 8 accumulator
 // tiles, rows dk) and v_new[:, cols] (C x 16, 8 tiles, rows tokens). Per chunk:
 //   P1  v_new = u + (-w) S             A: -w (LDS, rows tokens), B: S from the accumulators
@@ -1750,6 +1753,273 @@ __global__ __launch_bounds__(512) void k_scan_fwd_split(GdnArgs A) {
       if (nx != n) put_gates(nx);  // (the last step's would rewrite the carry being read)
       __syncthreads();
     }
+  }
+}
+
+// ---------------------------------------------------------------- k_scan_fwd_quad
+// The forward scan at C = D = 128 in the bf16 modes: k_scan_fwd_split's two products per chunk on
+// four compute waves, one per SIMD. Wave w owns 16 value columns (w % 2) and half the rows (w / 2)
+// of both products: 64 dk rows of S and 64 token rows of v_new, 4 accumulator tiles each. A
+// product's B operand needs the other product's rows of both halves: each wave converts its own
+// two 32-row steps to fragments (acc_pair_to_b) and leaves them in LDS for its partner (w ^ 2) as
+// they lie, one 16-byte write per lane and plane. Four loader waves, one per SIMD, stage -w and k
+// by rows, each value split once and written 8 bytes at a time: the A fragments of P1 are 16-byte
+// reads of -w's rows, those of P2 (k^T) transposing reads of k's rows (ds_read_b64_tr_b16), so
+// nothing is transposed on its way into LDS (swz_at spreads both kinds of read over the banks).
+// Two barriers per chunk; k and w are loaded a whole chunk step ahead. The order of every
+// accumulation is k_scan_fwd_split's: the same results bit for bit.
+//
+// What bounds it is the CU's memory pipe: 160 KB go through it per step (k and w, 64 KB each, read
+// by every one of a head's four workgroups) with about 56 KB in flight, beside 4 K cycles of LDS
+// per step of about 10 K. Measured against the two-wave form (which transposed k into LDS and left
+// its chunk index in vector registers): one row of 8192 tokens, 32 heads (128 workgroups) 312 -> 281 us; two
+// rows of 2048, 16 heads 76 -> 58 us; 0.8B layer shape (256 workgroups) 185 -> 171 us. Eight
+// loader waves (168 registers: spills) took 354 us there, w split ahead by k_chunk 292, lines touched three chunks
+// ahead by the compute waves 314.
+typedef short i16x4 __attribute__((ext_vector_type(4)));
+// the four values of one column (lane % 16) from four rows, 16 columns by four rows per 16 lanes
+// (lane l's address: row (l % 16) / 4, columns 4 (l % 4) .. + 3)
+__device__ __forceinline__ i16x4 lds_read_tr(const uint16_t* p) {
+  typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)p);
+}
+// the A fragment (row index: the column, contraction: 8 rows) from the lane's addresses of rows
+// 0-3 and 4-7
+__device__ __forceinline__ bf16x8 tr_frag(const uint16_t* lo, const uint16_t* hi) {
+  const i16x4 x = lds_read_tr(lo), y = lds_read_tr(hi);
+  const __attribute__((ext_vector_type(8))) short v = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+  return __builtin_bit_cast(bf16x8, v);
+}
+
+template <int PI, int PS>
+__global__ __launch_bounds__(512) void k_scan_fwd_quad(GdnArgs A) {
+  static_assert(PI != P_F32 && PS != P_F32, "the bf16 modes");
+  constexpr int C = 128, D = 128, DVT = 32, NT = 512;
+  constexpr int PL = C * D;                            // elements of a plane
+  constexpr int NW = PS == P_BF16X3 ? 2 : 1, NK = PI == P_BF16X3 ? 2 : 1;  // planes of -w and k
+  __shared__ __align__(16) uint16_t sW[NW * PL];       // -w [token][dk], swizzled
+  __shared__ __align__(16) uint16_t sK[NK * PL];       // k [token][dk], swizzled
+  // B fragments on their way to the partner: S's from wave w in box w ^ 2, v_new's in box w. A
+  // box is read by one wave per phase, the one that writes it next: no barrier in between.
+  __shared__ __align__(16) uint4 box[4][2][2][64];     // [box][32-row step][plane][lane]
+  __shared__ __align__(16) float skws[2][C];           // kws per token, by chunk parity
+  __shared__ float scarry[2];
+  __shared__ int red[NT / 64];
+  GDN_POISON_LDS(sW, sK, box, skws, scarry, red);
+  const ScanIx ix(A);
+  const int tile = ix.tile, bh = ix.bh, part = ix.part;
+  const int h = bh % A.H, b = bh / A.H, hk = h / A.ratio;
+  const int j0 = tile * DVT;
+  const int w = wave(), l = lane();
+  const int n0 = part_start<C, NT, true>(A, b, (int)((long)part * A.N / A.parts), red);
+  const int n1 = part_start<C, NT, true>(A, b, (int)((long)(part + 1) * A.N / A.parts), red);
+  if (n0 >= n1) return;
+  const int nb = n0 > 0 ? n0 - 1 : 0;
+  if (w < 4) {  // ---- compute waves
+    const int rh = w >> 1;                  // the wave's 64 rows of both products
+    const int col = j0 + 16 * (w & 1);      // its first value column
+    const int r = l & 15, g = l >> 4;
+    // A fragments of -w: row 64 rh + 16 t + r, units 4 s + g (swizzled: the row's low bits are r's)
+    const uint16_t* wp = sW + (64 * rh + r) * D;
+    const int wu = (g ^ swz(r)) << 3;       // s even; s odd: ^ 32
+    // of k^T: dk column 64 rh + 16 t + r, tokens 32 s + 8 g .. + 7
+    const uint16_t* kp[2];                  // rows 0-3 and 4-7 of the eight, less the unit
+    int ku[2][4];                           // the unit of column tile t there
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int row = 8 * g + (r >> 2) + 4 * e;
+      kp[e] = sK + row * D + 4 * (r & 1);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) ku[e][t] = ((8 * rh + 2 * t + ((r & 3) >> 1)) ^ swz(row)) << 3;
+    }
+    f32x4 accS[4];  // S[64 rh + 16 t + 4 (lane/16) + rr][col + lane % 16]
+    f32x4 accV[4];  // v_new[64 rh + 16 t + 4 (lane/16) + rr][col + lane % 16]
+    zero(accS);
+    if (n0 == 0 && A.init_state) {
+      const float* s0 = A.init_state + (size_t)bh * D * D + col + acc_col();
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) accS[t][rr] = s0[(size_t)(64 * rh + 16 * t + acc_row(rr)) * D];
+    }
+    float u[4][4];  // u at v_new's layout, loaded a chunk ahead
+    auto fetch_u = [&](int n) {
+      const float* ug = A.uu + hoff(A, b, h, A.H, n, C, D) + col;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) u[t][rr] = *lane_ptr(ug, 64 * rh + 16 * t + acc_row(rr), D, acc_col());
+    };
+    // the wave's own two steps of a B operand from its accumulator tiles, to the partner's box
+    auto post = [&](auto& f, const f32x4 (&acc)[4], int bx, const float* scale) {
+      constexpr int P = sizeof(f[0]) == sizeof(Frag<P_BF16X3>) ? P_BF16X3 : P_BF16;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        float v[8];
+        acc_pair_to_b(acc[2 * j], acc[2 * j + 1], v);
+        if (scale) {  // the lane's 8 contraction rows
+          const float4 s0 = *reinterpret_cast<const float4*>(scale + 64 * rh + 32 * j + 8 * g);
+          const float4 s1 = *reinterpret_cast<const float4*>(scale + 64 * rh + 32 * j + 8 * g + 4);
+          v[0] *= s0.x; v[1] *= s0.y; v[2] *= s0.z; v[3] *= s0.w;
+          v[4] *= s1.x; v[5] *= s1.y; v[6] *= s1.z; v[7] *= s1.w;
+        }
+        f[j] = make_frag<P>(v);
+        box[bx][j][0][l] = __builtin_bit_cast(uint4, f[j].hi);
+        if constexpr (P == P_BF16X3) box[bx][j][1][l] = __builtin_bit_cast(uint4, f[j].lo);
+      }
+    };
+    auto take = [&](auto& f, int bx) {
+      constexpr int P = sizeof(f[0]) == sizeof(Frag<P_BF16X3>) ? P_BF16X3 : P_BF16;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        f[j].hi = __builtin_bit_cast(bf16x8, box[bx][j][0][l]);
+        if constexpr (P == P_BF16X3) f[j].lo = __builtin_bit_cast(bf16x8, box[bx][j][1][l]);
+      }
+    };
+    auto frag_w = [&](Frag<PS> (&fa)[4], int s) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const uint16_t* p = wp + 16 * t * D + ((wu ^ (32 * (s & 1))) + 64 * (s >> 1));
+        fa[t].hi = *reinterpret_cast<const bf16x8*>(p);
+        if constexpr (PS == P_BF16X3) fa[t].lo = *reinterpret_cast<const bf16x8*>(p + PL);
+      }
+    };
+    auto frag_k = [&](Frag<PI> (&fa)[4], int s) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const uint16_t *p0 = kp[0] + ku[0][t] + 32 * s * D, *p1 = kp[1] + ku[1][t] + 32 * s * D;
+        fa[t].hi = tr_frag(p0, p1);
+        if constexpr (PI == P_BF16X3) fa[t].lo = tr_frag(p0 + PL, p1 + PL);
+      }
+    };
+    fetch_u(nb);
+    for (int n = nb; n < n1; ++n) {
+      const bool emit = n >= n0;  // the replayed chunk n0 - 1 only rebuilds the state
+      Frag<PS> own[2], other[2], fw[2][4];
+      post(own, accS, w ^ 2, nullptr);
+      if (emit) {
+        StateT<PS>* sg = states_ptr<PS>(A) + ((size_t)bh * A.N + n) * D * D + (size_t)(64 * rh) * D + col;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          if constexpr (sizeof(StateT<PS>) == 2) {  // and the final state's fp32 source
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr)
+              stf(sg + (unsigned)((16 * t + acc_row(rr)) * D + acc_col()), accS[t][rr]);
+            if (n == A.N - 1 && A.s_last)
+              st_tile(A.s_last + (size_t)bh * D * D + (size_t)(64 * rh + 16 * t) * D + col, D, accS[t]);
+          } else {
+            st_tile(sg + 16 * t * D, D, accS[t]);
+          }
+        }
+      }
+      __syncthreads();  // chunk n's -w and gates staged, the S fragments posted
+      frag_w(fw[0], 0);
+      take(other, w);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) accV[t] = f32x4{u[t][0], u[t][1], u[t][2], u[t][3]};
+      fetch_u(n + 1 < n1 ? n + 1 : n);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {  // P1: v_new = u + (-w) S
+        if (s + 1 < 4) frag_w(fw[(s + 1) & 1], s + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const Frag<PS> fb = (s >> 1) == rh ? own[s & 1] : other[s & 1];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) mma<PS>(accV[t], fw[s & 1][t], fb);
+      }
+      Frag<PI> vown[2], vother[2], fk[2][4];
+      post(vown, accV, w, skws[n & 1]);
+      if (emit) {
+        float* vg = A.vnew + hoff(A, b, h, A.H, n, C, D) + (size_t)(64 * rh) * D + col;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) st_tile(vg + 16 * t * D, D, accV[t]);
+      }
+      __syncthreads();  // chunk n's k staged, the v_new fragments posted
+      frag_k(fk[0], 0);
+      take(vother, w ^ 2);
+      const float carry = scarry[n & 1];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) accS[t] *= carry;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {  // P2: S = carry S + k^T (kws v_new)
+        if (s + 1 < 4) frag_k(fk[(s + 1) & 1], s + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const Frag<PI> fb = (s >> 1) == rh ? vown[s & 1] : vother[s & 1];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) mma<PI>(accS[t], fk[s & 1][t], fb);
+      }
+    }
+    return;
+  }
+  // ---- loader waves
+  const int lt = (int)threadIdx.x - 256;
+  float4 wr[16], kr[16];  // 4096 float4 slots each
+  int gs, gsc, gprev;
+  float gg, gl, ggc, glc;
+  // slot it of a thread: row lt / 32 + 8 it, columns 4 (lt % 32) .. + 3 (the row's swizzle is the
+  // same in all of them)
+  const int row0 = lt >> 5, c4 = lt & 31;
+  const unsigned goff = row0 * D + 4 * c4;
+  const int soff = swz_at(row0, c4 >> 1) + 4 * (c4 & 1);
+  auto fetch = [&](float4 (&x)[16], const float* src) {
+#pragma unroll
+    for (int it = 0; it < 16; ++it) x[it] = *reinterpret_cast<const float4*>(src + 8 * it * D + goff);
+  };
+  auto fetch_w = [&](int n) { fetch(wr, A.ww + hoff(A, b, h, A.H, n, C, D)); };
+  auto fetch_k = [&](int n) { fetch(kr, A.kn + hoff(A, b, hk, A.Hk, n, C, D)); };
+  // rows as split planes (sgn: the sign of the staged values)
+  auto put = [&](uint16_t* dst, const float4 (&x)[16], auto planes, float sgn) {
+#pragma unroll
+    for (int it = 0; it < 16; ++it) {
+      uint16_t* p = dst + soff + 8 * it * D;
+      const float a = sgn * x[it].x, c = sgn * x[it].y, d = sgn * x[it].z, e = sgn * x[it].w;
+      if constexpr (decltype(planes)::value == 2) {
+        const Split2 f = split2(a, c), g = split2(d, e);
+        *reinterpret_cast<uint2*>(p) = make_uint2(f.hi, g.hi);
+        *reinterpret_cast<uint2*>(p + PL) = make_uint2(f.lo, g.lo);
+      } else {
+        *reinterpret_cast<uint2*>(p) = make_uint2(pack2(a, c), pack2(d, e));
+      }
+    }
+  };
+  auto put_w = [&]() { put(sW, wr, std::integral_constant<int, NW>(), -1.f); };
+  auto put_k = [&]() { put(sK, kr, std::integral_constant<int, NK>(), 1.f); };
+  // the gates of chunk n: token lt's segment and gamma (lt < C), the chunk's last token and the
+  // token before it
+  auto fetch_g = [&](int n) {
+    const size_t tb = (size_t)b * A.Tp + (size_t)n * C, th = (size_t)(b * A.H + h) * A.Tp + (size_t)n * C;
+    const int t = lt % C;
+    gs = A.segp[tb + t];
+    gg = A.gam[th + t];
+    gl = A.gaml[th + t];
+    gsc = A.segp[tb + C - 1];
+    ggc = A.gam[th + C - 1];
+    glc = A.gaml[th + C - 1];
+    gprev = A.segp[n > 0 ? tb - 1 : tb];
+  };
+  auto put_gates = [&](int n) {  // kws and carry of chunk n into the parity buffers
+    const int before = (n == 0 && !A.init_state) ? -2 : gprev;
+    if (lt < C) skws[n & 1][lt] = gs == gsc ? expf((ggc - gg) + (glc - gl)) : 0.f;
+    if (lt == 0) scarry[n & 1] = gsc == before ? expf(ggc + glc) : 0.f;
+  };
+  auto upto = [&](int n) { return n < n1 ? n : n1 - 1; };  // past the range: its last chunk again (unused)
+  fetch_g(nb);
+  fetch_w(nb);
+  fetch_k(nb);
+  put_gates(nb);
+  put_w();
+  fetch_g(upto(nb + 1));
+  fetch_w(upto(nb + 1));
+  __syncthreads();
+  for (int n = nb;; ++n) {
+    put_k();  // k of chunk n, during P1
+    fetch_k(upto(n + 1));
+    __syncthreads();
+    if (n + 1 >= n1) break;
+    put_gates(n + 1);  // -w and the gates of the next chunk, during P2
+    put_w();
+    fetch_g(upto(n + 2));
+    fetch_w(upto(n + 2));
+    __syncthreads();
   }
 }
 
