@@ -176,6 +176,13 @@ def open_library(path: Path) -> ctypes.CDLL:
     return lib
 
 
+def current_stream(device: torch.device) -> int:
+    """The handle of torch's current stream on ``device`` (what current_stream(device).cuda_stream
+    gives, without building the Stream object: 2 us of a 16 us decode step)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
 def check_status(status: int) -> None:
     if status != 0:
         raise GdnLibraryError(status, load().tjev_gdn_last_error().decode())

@@ -19,6 +19,7 @@ CPU tensor, the operator raises.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 
 import torch
@@ -162,9 +163,11 @@ class GdnPlan:
         self.fwd_bytes = self.lib.tjev_gdn_workspace_bytes(ctypes.byref(self.params), 0)
         self.bwd_bytes = self.lib.tjev_gdn_workspace_bytes(ctypes.byref(self.params), 1)
 
+        self._normed_bytes: dict[bool, int] = {}
+
     @staticmethod
     def _stream(device: torch.device) -> int:
-        return torch.cuda.current_stream(device).cuda_stream
+        return _lib.current_stream(device)
 
     def workspace(self, backward: bool, device) -> torch.Tensor:
         return torch.empty(self.bwd_bytes if backward else self.fwd_bytes, dtype=torch.uint8, device=device)
@@ -207,7 +210,10 @@ class GdnPlan:
         _lib.check_status(status)
 
     def normed_bwd_bytes(self, norm_weight_grad: bool) -> int:
-        return int(self.lib.tjev_gdn_workspace_bytes_normed(ctypes.byref(self.params), int(norm_weight_grad)))
+        want = bool(norm_weight_grad)
+        if want not in self._normed_bytes:
+            self._normed_bytes[want] = int(self.lib.tjev_gdn_workspace_bytes_normed(ctypes.byref(self.params), int(want)))
+        return self._normed_bytes[want]
 
     def backward_normed(self, qkv, a, b, a_log, dt_bias, conv_w, seg, residuals, out, gate, norm_weight,
                         eps: float, d_y, d_qkv, d_a, d_b, d_a_log, d_dt_bias, d_conv_w, d_gate, d_norm_weight,
@@ -229,6 +235,21 @@ class GdnPlan:
             _ptr(dt_bias), _ptr(conv_w), _ptr(seg), _ptr(residuals), _ptr(d_out), _ptr(d_qkv), _ptr(d_a),
             _ptr(d_b), _ptr(d_a_log), _ptr(d_dt_bias), _ptr(d_conv_w), _ptr(workspace), workspace.numel())
         _lib.check_status(status)
+
+
+@functools.lru_cache(maxsize=256, typed=True)
+def _plan(lib, batch, length, key_heads, key_dim, value_heads, value_dim, taps, chunk, io_dtype, gate_dtype, precision,
+          inverse, heads_per_step, residuals, qk_dtype=None) -> GdnPlan:
+    """The plan of one problem shape on the library in use (``lib``, part of the key): a program
+    calls the operators on few shapes many times, and a plan's checks and size queries (9 library
+    calls) depend on these values alone. Plans are never changed once built, so calls and
+    threads share them."""
+    plan = GdnPlan(batch=batch, length=length, key_heads=key_heads, key_dim=key_dim, value_heads=value_heads,
+                   value_dim=value_dim, taps=taps, chunk=chunk, io_dtype=io_dtype, gate_dtype=gate_dtype,
+                   precision=precision, inverse=inverse, heads_per_step=heads_per_step, residuals=residuals)
+    if qk_dtype is not None:
+        plan.params.qk_dtype = _DTYPES[qk_dtype]
+    return plan
 
 
 class _Core(torch.autograd.Function):
@@ -381,6 +402,12 @@ class _CoreCont(torch.autograd.Function):
 def _check(precision, inverse, chunk, width, key_heads, key_dim, value_heads, value_dim, heads_per_step,
            conv_weight):
     """gdn_megakernel's checks, in its order and wording (pallas_tpu_mega.py:597-615)."""
+    return _check_values(precision, inverse, chunk, width, key_heads, key_dim, value_heads, value_dim, heads_per_step,
+                         None if conv_weight is None else conv_weight.shape[0])
+
+
+@functools.lru_cache(maxsize=256, typed=True)
+def _check_values(precision, inverse, chunk, width, key_heads, key_dim, value_heads, value_dim, heads_per_step, taps):
     if precision not in PRECISIONS:
         raise ValueError(f"precision in {PRECISIONS}")
     if inverse not in INVERSE_BLOCKS:
@@ -395,7 +422,7 @@ def _check(precision, inverse, chunk, width, key_heads, key_dim, value_heads, va
     hb = heads_per_block(value_heads, ratio, heads_per_step or 8)
     if 3 * hb > LANES:
         raise ValueError(f"at most 42 heads per step, not {hb}")
-    taps = 1 if conv_weight is None else conv_weight.shape[0]
+    taps = 1 if taps is None else taps
     if not 1 <= taps <= 5:
         raise ValueError(f"conv kernel of {taps} taps: the megakernel supports 1..5")
     return taps
@@ -453,10 +480,9 @@ def gdn_megakernel(qkv: torch.Tensor, a: torch.Tensor, b: torch.Tensor, a_log: t
                                   precision=precision, inverse=inverse, heads_per_step=heads_per_step,
                                   residuals=residuals, initial_state=initial_state, initial_conv=initial_conv,
                                   output_final_state=output_final_state)
-    plan = GdnPlan(batch=batch, length=length, key_heads=key_heads, key_dim=key_dim, value_heads=value_heads,
-                   value_dim=value_dim, taps=0 if conv_weight is None else taps, chunk=chunk,
-                   io_dtype=qkv.dtype, gate_dtype=a.dtype, precision=precision, inverse=inverse,
-                   heads_per_step=heads_per_step, residuals=residuals)
+    plan = _plan(_lib.load(), batch, length, key_heads, key_dim, value_heads, value_dim,
+                 0 if conv_weight is None else taps, chunk, qkv.dtype, a.dtype, precision, inverse, heads_per_step,
+                 residuals)
     b = b.to(a.dtype)
     conv_w = None if conv_weight is None else conv_weight.to(torch.float32).contiguous()
     args = (qkv.contiguous(), a.contiguous(), b.contiguous(), a_log.to(torch.float32).contiguous(),
@@ -507,10 +533,9 @@ def gdn_megakernel_normed(qkv: torch.Tensor, a: torch.Tensor, b: torch.Tensor, a
                              key_dim=key_dim, value_heads=value_heads, value_dim=value_dim, chunk=chunk,
                              precision=precision, inverse=inverse, heads_per_step=heads_per_step, residuals=residuals)
         return _norm_any_dim(out, gate, norm_weight, eps, segment_ids)
-    plan = GdnPlan(batch=batch, length=length, key_heads=key_heads, key_dim=key_dim, value_heads=value_heads,
-                   value_dim=value_dim, taps=0 if conv_weight is None else taps, chunk=chunk,
-                   io_dtype=qkv.dtype, gate_dtype=a.dtype, precision=precision, inverse=inverse,
-                   heads_per_step=heads_per_step, residuals=residuals)
+    plan = _plan(_lib.load(), batch, length, key_heads, key_dim, value_heads, value_dim,
+                 0 if conv_weight is None else taps, chunk, qkv.dtype, a.dtype, precision, inverse, heads_per_step,
+                 residuals)
     b = b.to(a.dtype)
     conv_w = None if conv_weight is None else conv_weight.to(torch.float32).contiguous()
     return _CoreNormed.apply(plan, qkv.contiguous(), a.contiguous(), b.contiguous(),

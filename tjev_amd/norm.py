@@ -31,7 +31,7 @@ def _params(tokens: int, heads: int, dim: int, dtype: torch.dtype, eps: float) -
 
 
 def _stream(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return ctypes.c_void_p(_lib.current_stream(device))
 
 
 def norm_forward(p: _lib.NormParams, x, gate, weight, seg, y) -> None:

@@ -14,12 +14,13 @@ belongs to; a new request starts from a fresh prefill.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 
 import torch
 
 from . import _lib
-from .gdn import GdnPlan, _check, _ptr, merge_value_cols, pad_qkv, run_dim, unpad_qkv, value_cols, value_groups
+from .gdn import _check, _plan, _ptr, merge_value_cols, pad_qkv, run_dim, unpad_qkv, value_cols, value_groups
 
 _DTYPES = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16}
 
@@ -67,9 +68,8 @@ def gdn_prefill(qkv, a, b, a_log, dt_bias, conv_weight, segment_ids, *, key_head
         if conv_state is not None:
             conv_state = unpad_qkv(conv_state, key_heads, key_dim, value_heads, value_dim, run)
         return out.contiguous(), state[:, :, :key_dim, :value_dim].contiguous(), conv_state
-    plan = GdnPlan(batch=batch, length=length, key_heads=key_heads, key_dim=key_dim, value_heads=value_heads,
-                   value_dim=value_dim, taps=0 if conv_weight is None else taps, chunk=chunk, io_dtype=qkv.dtype,
-                   gate_dtype=a.dtype, precision=precision, inverse=inverse, heads_per_step=heads_per_step)
+    plan = _plan(_lib.load(), batch, length, key_heads, key_dim, value_heads, value_dim,
+                 0 if conv_weight is None else taps, chunk, qkv.dtype, a.dtype, precision, inverse, heads_per_step, "states")
     dev = qkv.device
     qkv, a, seg = qkv.contiguous(), a.contiguous(), segment_ids.to(torch.int32).contiguous()
     b = b.to(a.dtype).contiguous()
@@ -96,6 +96,18 @@ def gdn_prefill(qkv, a, b, a_log, dt_bias, conv_weight, segment_ids, *, key_head
     return out, state, conv_state
 
 
+@functools.lru_cache(maxsize=256, typed=True)
+def _decode_params(batch, key_heads, key_dim, value_heads, value_dim, taps, io_dtype, gate_dtype):
+    """The library's view of a decode step's shape (a reference to the struct; never changed)."""
+    return ctypes.byref(_lib.Params(batch, 1, key_heads, key_dim, value_heads, value_dim, taps, 64, _DTYPES[io_dtype],
+                                    _DTYPES[gate_dtype], 1, 0, 0, 0))
+
+
+@functools.lru_cache(maxsize=256, typed=True)
+def _decode_dims(key_dim, value_dim):
+    return value_groups(key_dim, value_dim), run_dim(key_dim, value_dim)
+
+
 def gdn_decode_step(qkv, a, b, a_log, dt_bias, conv_weight, conv_state, state, *, key_heads: int, key_dim: int,
                     value_heads: int, value_dim: int, inplace: bool = False):
     """One token per row: qkv [B, W] (raw; post-conv for ``conv_weight`` None), a, b [B, H],
@@ -115,7 +127,7 @@ def gdn_decode_step(qkv, a, b, a_log, dt_bias, conv_weight, conv_state, state, *
         raise ValueError(f"state must be fp32 [{batch}, {value_heads}, {key_dim}, {value_dim}]")
     if taps > 1 and (conv_state is None or conv_state.shape != (batch, taps - 1, width)):
         raise ValueError(f"conv_state must be [{batch}, {taps - 1}, {width}]")
-    groups = value_groups(key_dim, value_dim)
+    groups, run = _decode_dims(key_dim, value_dim)
     if groups is not None:  # value heads wider than 128: groups of value columns (gdn_megakernel's split)
         cut = lambda x, c, w: None if x is None else value_cols(  # noqa: E731
             x, key_heads, key_dim, value_heads, value_dim, c, w)
@@ -131,7 +143,6 @@ def gdn_decode_step(qkv, a, b, a_log, dt_bias, conv_weight, conv_state, state, *
             state.copy_(st)
             st = state
         return out, hist_out, st
-    run = run_dim(key_dim, value_dim)
     if run is None:
         raise ValueError(f"key dims up to 128: this build's kernels cannot hold Dk={key_dim}, Dv={value_dim}")
     if run != key_dim or run != value_dim:  # zero-padded heads (gdn_megakernel's padded route)
@@ -148,15 +159,15 @@ def gdn_decode_step(qkv, a, b, a_log, dt_bias, conv_weight, conv_state, state, *
         hist_out = None if hist_out is None else unpad_qkv(hist_out, key_heads, key_dim, value_heads, value_dim, run)
         return out.contiguous(), hist_out, st.contiguous() if not inplace else st
     lib = _lib.load()
-    p = _lib.Params(batch, 1, key_heads, key_dim, value_heads, value_dim, taps, 64, _DTYPES[qkv.dtype],
-                    _DTYPES[a.dtype], 1, 0, 0, 0)
     dev = qkv.device
     qkv, a = qkv.contiguous(), a.contiguous()
-    b = b.to(a.dtype).contiguous()
-    a_log, dt_bias = a_log.to(torch.float32).contiguous(), dt_bias.to(torch.float32).contiguous()
-    conv_w = None if conv_weight is None else conv_weight.to(torch.float32).contiguous()
-    hist = None if taps <= 1 else conv_state.to(qkv.dtype).contiguous()
-    hist_out = None if taps <= 1 else torch.empty_like(hist)
+    b = (b if b.dtype == a.dtype else b.to(a.dtype)).contiguous()
+    a_log, dt_bias, conv_w = (x if x is None or (x.dtype == torch.float32 and x.is_contiguous())
+                              else x.to(torch.float32).contiguous() for x in (a_log, dt_bias, conv_weight))
+    hist = hist_out = None
+    if taps > 1:
+        hist = (conv_state if conv_state.dtype == qkv.dtype else conv_state.to(qkv.dtype)).contiguous()
+        hist_out = torch.empty_like(hist)
     if inplace and (not state.is_contiguous() or state.data_ptr() % 16):
         raise ValueError("inplace: the state must be a contiguous, 16-byte aligned fp32 tensor (a copy would "
                          "leave the caller's cache unchanged)")
@@ -164,8 +175,8 @@ def gdn_decode_step(qkv, a, b, a_log, dt_bias, conv_weight, conv_state, state, *
     state_out = state if inplace else torch.empty_like(state)
     out = torch.empty((batch, value_heads, value_dim), dtype=qkv.dtype, device=dev)
     status = lib.tjev_gdn_decode_step(
-        ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream), _ptr(qkv), _ptr(a), _ptr(b),
-        _ptr(a_log), _ptr(dt_bias), _ptr(conv_w), _ptr(hist), _ptr(state), _ptr(out), _ptr(hist_out),
-        _ptr(state_out))
+        _decode_params(batch, key_heads, key_dim, value_heads, value_dim, taps, qkv.dtype, a.dtype),
+        _lib.current_stream(dev), qkv.data_ptr(), a.data_ptr(), b.data_ptr(), a_log.data_ptr(), dt_bias.data_ptr(),
+        _ptr(conv_w), _ptr(hist), state.data_ptr(), out.data_ptr(), _ptr(hist_out), state_out.data_ptr())
     _lib.check_status(status)
     return out, hist_out, state_out

@@ -18,7 +18,7 @@ import ctypes
 import torch
 
 from . import _lib
-from .gdn import INVERSE_BLOCKS, LANES, PRECISIONS, GdnPlan, _ptr, heads_per_block, run_dim, value_groups
+from .gdn import INVERSE_BLOCKS, LANES, PRECISIONS, GdnPlan, _plan, _ptr, heads_per_block, run_dim, value_groups
 
 _DTYPES = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16}
 
@@ -152,10 +152,8 @@ def chunk_gated_delta_rule_v2(q, k, v, g, beta, segment_ids=None, *, chunk: int 
     if segment_ids is None:
         segment_ids = torch.ones((batch, length), dtype=torch.int32, device=v.device)
     qk_dtype = q.dtype if q.dtype in _DTYPES else torch.float32
-    plan = GdnPlan(batch=batch, length=length, key_heads=kheads, key_dim=dk, value_heads=heads, value_dim=dv, taps=0,
-                   chunk=chunk, io_dtype=v.dtype, gate_dtype=g.dtype if g.dtype in _DTYPES else torch.float32,
-                   precision=precision, inverse=inverse, heads_per_step=heads_per_step, residuals=residuals)
-    plan.params.qk_dtype = _DTYPES[qk_dtype]
+    plan = _plan(_lib.load(), batch, length, kheads, dk, heads, dv, 0, chunk, v.dtype,
+                 g.dtype if g.dtype in _DTYPES else torch.float32, precision, inverse, heads_per_step, residuals, qk_dtype)
     gd = torch.bfloat16 if plan.params.gate_dtype == _lib.BF16 else torch.float32
     args = (q.to(qk_dtype).contiguous(), k.to(qk_dtype).contiguous(), v.contiguous(), g.to(gd).contiguous(),
             beta.to(gd).contiguous(), segment_ids.to(torch.int32).contiguous())
