@@ -216,6 +216,22 @@ int tjev_gdn_decode_step(const tjev_gdn_params* p, void* stream, const void* qkv
                          const float* conv_w, const void* conv_state, const float* state,
                          void* out, void* conv_state_out, float* state_out);
 
+/* The merged projections of the LoRA-adapted layer (the reference's _merge, lora.py:284-295):
+ * merged [in, out] bf16 = round(w + scale * a b), w [in, out] bf16, a [in, rank] and b [rank, out]
+ * fp32, rounded to bf16 before their product, which accumulates in fp32. n projections (up to
+ * TJEV_GDN_MAX_MERGE) in one launch; out in multiples of 8, one rank for all of 32, 64, 96 or
+ * 128; every tensor 16-byte aligned and contiguous; merged aliases none of the inputs. */
+#define TJEV_GDN_MAX_MERGE 8
+typedef struct tjev_gdn_merge {
+  const void* w;
+  const float* a;
+  const float* b;
+  void* merged;
+  int32_t in, out, rank;
+  float scale;
+} tjev_gdn_merge;
+int tjev_gdn_lora_merge(const tjev_gdn_merge* projections, int n, void* stream);
+
 /* The v2 operator (tjev's chunk_gated_delta_rule_v2, pallas_tpu_v2.py:541-582, behind
  * gdn_impl=pallas_tpu_v2): the same chunked delta rule on given q, k [B, T, Hk, Dk] (qk_dtype;
  * used as given: the model passes l2norm(q) * Dk^-1/2 and l2norm(k)), v [B, T, H, Dv]

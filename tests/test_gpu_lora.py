@@ -1,0 +1,48 @@
+"""The merged projections' kernel (tjev_gdn_lora_merge) at the edges of its tiles (rows and columns
+below, at and past a 16-row strip, a 256-row and a 128-column tile), every rank, several projections in one
+launch: round(w + s a b) with a and b rounded to bf16, against fp64 on the same rounded values.
+The kernel's fp32 sum is within 2^-24 (rank + 2) of sum |a b| s + |w| of the exact one, so a result
+is the bf16 rounding of a value that far off: half a bf16 spacing past it (bf16 keeps 8 bits: the
+spacing at |v| in [2^e, 2^(e+1)) is 2^(e-7), half of it at most 2^-8 |v|)."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rank", [32, 64, 96, 128])
+@pytest.mark.parametrize("shapes", [[(1, 8)], [(15, 136), (17, 128), (16, 120)], [(257, 256), (255, 32), (256, 264), (2560, 64)]])
+def test_merge_matches_fp64(rank, shapes):
+    from tjev_amd.block import _merge_all
+
+    gen = torch.Generator().manual_seed(rank)
+    rn = lambda *s: torch.randn(s, generator=gen)  # noqa: E731
+    ws = [rn(i, o).to(torch.bfloat16) for i, o in shapes]
+    a_s, b_s = [rn(i, rank) * rank ** -0.5 for i, o in shapes], [rn(rank, o) * 0.3 for i, o in shapes]
+    scales = [0.5 + n for n in range(len(shapes))]
+    print(f"merge rank={rank} {shapes}", flush=True)
+    got = _merge_all([w.cuda() for w in ws], [a.cuda() for a in a_s], [b.cuda() for b in b_s], scales, torch.bfloat16)
+    torch.cuda.synchronize()
+    for w, a, b, s, y in zip(ws, a_s, b_s, scales, got):
+        a, b, w = a.bfloat16().double(), b.bfloat16().double(), w.double()
+        want = w + s * (a @ b)
+        room = 2.0 ** -24 * (rank + 2) * (w.abs() + s * (a.abs() @ b.abs()))
+        err = (y.double().cpu() - want).abs()
+        assert bool((err <= 2.0 ** -8 * (want.abs() + room) + room).all()), float((err / want.abs()).max())
+
+
+def test_merge_refuses_what_it_does_not_hold():
+    from tjev_amd import _lib
+
+    lib = _lib.load()
+    t = torch.zeros(64, 64, device="cuda")
+    p = t.data_ptr()
+    ok = dict(w=p, a=p, b=p, merged=p, inputs=16, outputs=16, rank=32, scale=1.0)
+    for bad, status in ((dict(outputs=12), 2), (dict(rank=48), 2), (dict(rank=160), 2), (dict(inputs=0), 1), (dict(w=None), 1),
+                        (dict(b=p + 4), 1)):
+        assert lib.tjev_gdn_lora_merge((_lib.Merge * 1)(_lib.Merge(**{**ok, **bad})), 1, None) == status, bad
+    assert lib.tjev_gdn_lora_merge((_lib.Merge * 9)(*[_lib.Merge(**ok)] * 9), 9, None) == 1
+    assert lib.tjev_gdn_lora_merge(None, 1, None) == 1

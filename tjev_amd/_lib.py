@@ -37,6 +37,7 @@ EXPORTS = (
     "tjev_gdn_mega2_bwd_cont",
     "tjev_gdn_mega2_fwd_cont_noalloc",
     "tjev_gdn_decode_step",
+    "tjev_gdn_lora_merge",
     "tjev_gdn_v2_fwd",
     "tjev_gdn_v2_bwd",
     "tjev_gdn_v2_fwd_cont",
@@ -70,6 +71,17 @@ class NormParams(ctypes.Structure):
 
     _fields_ = [("tokens", ctypes.c_int64), ("heads", ctypes.c_int32), ("dim", ctypes.c_int32),
                 ("dtype", ctypes.c_int32), ("eps", ctypes.c_float)]
+
+
+class Merge(ctypes.Structure):
+    """tjev_gdn_merge"""
+
+    _fields_ = [("w", ctypes.c_void_p), ("a", ctypes.c_void_p), ("b", ctypes.c_void_p), ("merged", ctypes.c_void_p),
+                ("inputs", ctypes.c_int32), ("outputs", ctypes.c_int32), ("rank", ctypes.c_int32),
+                ("scale", ctypes.c_float)]
+
+
+MAX_MERGE = 8  # TJEV_GDN_MAX_MERGE
 
 
 class GdnLibraryError(RuntimeError):
@@ -147,6 +159,8 @@ def open_library(path: Path) -> ctypes.CDLL:
     lib.tjev_gdn_v2_bwd_cont.restype = i32
     lib.tjev_gdn_decode_step.argtypes = [pp, vp] + [vp] * 11
     lib.tjev_gdn_decode_step.restype = i32
+    lib.tjev_gdn_lora_merge.argtypes = [ctypes.POINTER(Merge), i32, vp]
+    lib.tjev_gdn_lora_merge.restype = i32
     lib.tjev_gdn_v2_fwd.argtypes = [pp, vp] + [vp] * 9 + [sz]
     lib.tjev_gdn_v2_fwd.restype = i32
     lib.tjev_gdn_v2_bwd.argtypes = [pp, vp] + [vp] * 14 + [sz]

@@ -21,6 +21,7 @@ import math
 
 import torch
 
+from . import _lib
 from .gdn import gdn_megakernel_normed
 
 
@@ -67,6 +68,29 @@ def _merge(w: torch.Tensor, a: torch.Tensor, b: torch.Tensor, s: float, dtype) -
     return (w.to(torch.float32) + s * _mm32(a, b)).to(dtype)
 
 
+def _merge_all(ws, a_s, b_s, scales, dtype) -> list[torch.Tensor]:
+    """``_merge`` of every projection of a group: one launch of the HIP library's merge kernel for bf16
+    weights and fp32 adapters of one rank of 32, 64, 96 or 128 (any number of inputs; outputs in
+    multiples of 8), contiguous and 16-byte aligned as parameters are; else one GEMM each. A GEMM
+    with W as its addend first copies W into its output and takes bf16 copies of both adapters:
+    168 us for the 4B layer's five projections against 51 (two launches)."""
+    rank = a_s[0].shape[1]
+    if (dtype == torch.bfloat16 and len(ws) <= _lib.MAX_MERGE and rank in (32, 64, 96, 128)
+            and all(w.is_cuda and w.dtype == dtype and a.dtype == b.dtype == torch.float32 and w.shape[1] % 8 == 0
+                    and a.device == b.device == w.device == ws[0].device
+                    and a.shape == (w.shape[0], rank) and b.shape == (rank, w.shape[1])
+                    and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (w, a, b))
+                    for w, a, b in zip(ws, a_s, b_s))):
+        outs = [torch.empty_like(w) for w in ws]
+        args = (_lib.Merge * len(ws))(*(
+            _lib.Merge(w.data_ptr(), a.data_ptr(), b.data_ptr(), o.data_ptr(), *w.shape, rank, s)
+            for w, a, b, o, s in zip(ws, a_s, b_s, outs, scales)))
+        with torch.cuda.device(ws[0].device):
+            _lib.check_status(_lib.load().tjev_gdn_lora_merge(args, len(ws), _lib.current_stream(ws[0].device)))
+        return outs
+    return [_merge(w, a, b, s, dtype) for w, a, b, s in zip(ws, a_s, b_s, scales)]
+
+
 class _MergedLoRA(torch.autograd.Function):
     """``_merged_matmuls`` (lora.py:303-369) for projections sharing the input x [N, in]:
     y_i = x W'_i, W'_i = (W_i + s_i A_i B_i) in the compute dtype, A_i and B_i rounded to it
@@ -77,7 +101,7 @@ class _MergedLoRA(torch.autograd.Function):
         n = len(scales)
         ws, a_s, b_s = params[:n], params[n:2 * n], params[2 * n:]
         dtype = x.dtype
-        merged = [_merge(w, a, b, s, dtype) for w, a, b, s in zip(ws, a_s, b_s, scales)]
+        merged = _merge_all(ws, a_s, b_s, scales, dtype)
         ys = tuple(x @ m for m in merged)
         ctx.scales = scales
         ctx.save_for_backward(x, *merged, *a_s, *b_s)

@@ -31,8 +31,8 @@ FLAGS = [
 ]
 
 
-# units built once: the C ABI, the gated RMSNorm and the decode step
-EXTRA_UNITS = ("gdn_api", "gdn_norm", "gdn_decode")
+# units built once: the C ABI, the gated RMSNorm, the decode step and the merged LoRA projections
+EXTRA_UNITS = ("gdn_api", "gdn_norm", "gdn_decode", "gdn_lora")
 # object files per (chunk, head dim) pair: the launch sequences with the small kernels (part 0),
 # then one per large kernel family (gdn_inst.hip's GDN_PART)
 PARTS = 6
