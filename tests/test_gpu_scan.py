@@ -1,4 +1,4 @@
-"""The forward scan at C = D = 128 (four compute waves in the bf16 modes): one chunk, a chunk's edge
+"""The forward scan at D = 128, chunks of 64 and 128 (four compute waves in the bf16 modes): one chunk, a chunk's edge
 and several chunks, states that start given or reset inside, before and after a chunk, rows that
 are split into ranges at those resets, and grouped heads, in every precision. Outputs and final
 state against the oracle's fp64 token recurrence: 1e-5 at "highest", 1e-4 at "high" (three bf16
@@ -17,10 +17,11 @@ pytestmark = pytest.mark.gpu
 TOL = {"highest": 1e-5, "high": 1e-4, "mixed": 3e-2, "bf16": 3e-2}
 
 
+@pytest.mark.parametrize("chunk", [64, 128])
 @pytest.mark.parametrize("precision", list(TOL))
 @pytest.mark.parametrize("length,cuts,fresh", [(1, None, True), (128, None, False), (129, [128], True), (300, [127], False),
                                                (700, [64, 128, 256, 500], True), (640, None, False)])
-def test_scan_fwd_matches_the_recurrence(precision, length, cuts, fresh):
+def test_scan_fwd_matches_the_recurrence(precision, chunk, length, cuts, fresh):
     from oracle.gdn_oracle import recurrent_gated_delta_rule
     from tjev_amd.testing import cut_segments
     from tjev_amd.v2 import chunk_gated_delta_rule_v2
@@ -37,8 +38,8 @@ def test_scan_fwd_matches_the_recurrence(precision, length, cuts, fresh):
     seg = torch.ones(b, length, dtype=torch.int32)
     if cuts:
         seg[1] = torch.from_numpy(cut_segments(length, cuts))
-    print(f"scan {precision} T={length} cuts={cuts} fresh={fresh}", flush=True)
-    out, state = chunk_gated_delta_rule_v2(*(x.cuda() for x in (q, k, v, g, beta, seg)), chunk=128, precision=precision,
+    print(f"scan {precision} C={chunk} T={length} cuts={cuts} fresh={fresh}", flush=True)
+    out, state = chunk_gated_delta_rule_v2(*(x.cuda() for x in (q, k, v, g, beta, seg)), chunk=chunk, precision=precision,
                                            initial_state=None if s0 is None else s0.cuda(), output_final_state=True)
     torch.cuda.synchronize()
     rep = [x.double().repeat_interleave(h // hk, 2) for x in (q, k)]

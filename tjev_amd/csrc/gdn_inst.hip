@@ -79,12 +79,16 @@ GDN_EACH_PAIR(GDN_CHUNK_FV)
 #endif
 // part 2: the scans
 #define GDN_SCAN_BWD(PI, PS, TIO) GDN_KW_2 __global__ void k_scan_bwd<GDN_C, GDN_D, kDVT, PI, PS, TIO>(GdnArgs);
-#if GDN_C == 128 && GDN_D == 128
+#if GDN_C >= 64 && GDN_D == 128  // the bf16 modes on four compute waves
 #define GDN_SCAN_FWD(PI, PS)
+#if GDN_C == 128
 GDN_KW_2 __global__ void k_scan_fwd_split<P_F32, P_F32>(GdnArgs);
-GDN_KW_2 __global__ void k_scan_fwd_quad<P_BF16X3, P_BF16X3>(GdnArgs);
-GDN_KW_2 __global__ void k_scan_fwd_quad<P_BF16, P_BF16>(GdnArgs);
-GDN_KW_2 __global__ void k_scan_fwd_quad<P_BF16X3, P_BF16>(GdnArgs);
+#else
+GDN_KW_2 __global__ void k_scan_fwd<GDN_C, GDN_D, kDVT, P_F32, P_F32>(GdnArgs);
+#endif
+GDN_KW_2 __global__ void k_scan_fwd_quad<GDN_C, P_BF16X3, P_BF16X3>(GdnArgs);
+GDN_KW_2 __global__ void k_scan_fwd_quad<GDN_C, P_BF16, P_BF16>(GdnArgs);
+GDN_KW_2 __global__ void k_scan_fwd_quad<GDN_C, P_BF16X3, P_BF16>(GdnArgs);
 #else
 #define GDN_SCAN_FWD(PI, PS) GDN_KW_2 __global__ void k_scan_fwd<GDN_C, GDN_D, kDVT, PI, PS>(GdnArgs);
 #endif
@@ -188,7 +192,7 @@ hipError_t run(const GdnArgs& A, hipStream_t st, int backward, const Timer* tm) 
       } else if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, true>), persist, dim3(C * 4));
       else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, false>), persist, dim3(C * 4));
     }
-    if constexpr (C == 128 && D == 128 && PI != P_F32) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_quad<PI, PS>), tiles, dim3(512));
+    if constexpr (C >= 64 && D == 128 && PI != P_F32) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_quad<C, PI, PS>), tiles, dim3(512));
     else if constexpr (C == 128 && D == 128) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_split<PI, PS>), tiles, dim3(512));
     else GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd<C, D, DVT, PI, PS>), tiles, dim3(NS));
     if (L.fuse_q) {
@@ -262,7 +266,7 @@ hipError_t run_v2(const GdnArgs& A, hipStream_t st, int backward, const Timer* t
       if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, true>), persist, dim3(C * 4));
       else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, false>), persist, dim3(C * 4));
     }
-    if constexpr (C == 128 && D == 128 && PI != P_F32) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_quad<PI, PS>), tiles, dim3(512));
+    if constexpr (C >= 64 && D == 128 && PI != P_F32) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_quad<C, PI, PS>), tiles, dim3(512));
     else if constexpr (C == 128 && D == 128) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_split<PI, PS>), tiles, dim3(512));
     else GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd<C, D, DVT, PI, PS>), tiles, dim3(NS));
     GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO>), persist, dim3(C * 4));

@@ -1757,11 +1757,11 @@ __global__ __launch_bounds__(512) void k_scan_fwd_split(GdnArgs A) {
 }
 
 // ---------------------------------------------------------------- k_scan_fwd_quad
-// The forward scan at C = D = 128 in the bf16 modes: k_scan_fwd_split's two products per chunk on
-// four compute waves, one per SIMD. Wave w owns 16 value columns (w % 2) and half the rows (w / 2)
-// of both products: 64 dk rows of S and 64 token rows of v_new, 4 accumulator tiles each. A
+// The forward scan at D = 128 and chunks of 64 and 128 in the bf16 modes: k_scan_fwd_split's two
+// products per chunk on four compute waves, one per SIMD. Wave w owns 16 value columns (w % 2) and
+// half the rows (w / 2) of both products: 64 dk rows of S and C/2 token rows of v_new. A
 // product's B operand needs the other product's rows of both halves: each wave converts its own
-// two 32-row steps to fragments (acc_pair_to_b) and leaves them in LDS for its partner (w ^ 2) as
+// 32-row steps to fragments (acc_pair_to_b) and leaves them in LDS for its partner (w ^ 2) as
 // they lie, one 16-byte write per lane and plane. Four loader waves, one per SIMD, stage -w and k
 // by rows, each value split once and written 8 bytes at a time: the A fragments of P1 are 16-byte
 // reads of -w's rows, those of P2 (k^T) transposing reads of k's rows (ds_read_b64_tr_b16), so
@@ -1773,7 +1773,8 @@ __global__ __launch_bounds__(512) void k_scan_fwd_split(GdnArgs A) {
 // by every one of a head's four workgroups) with about 56 KB in flight, beside 4 K cycles of LDS
 // per step of about 10 K. Measured against the two-wave form (which transposed k into LDS and left
 // its chunk index in vector registers): one row of 8192 tokens, 32 heads (128 workgroups) 312 -> 281 us; two
-// rows of 2048, 16 heads 76 -> 58 us; 0.8B layer shape (256 workgroups) 185 -> 171 us. Eight
+// rows of 2048, 16 heads 76 -> 58 us; 0.8B layer shape (256 workgroups) 185 -> 171 us; chunks of 64
+// against k_scan_fwd (two rows of 1777, 32 heads, segment cuts): 128 -> 90 us. Eight
 // loader waves (168 registers: spills) took 354 us there, w split ahead by k_chunk 292, lines touched three chunks
 // ahead by the compute waves 314.
 typedef short i16x4 __attribute__((ext_vector_type(4)));
@@ -1791,10 +1792,13 @@ __device__ __forceinline__ bf16x8 tr_frag(const uint16_t* lo, const uint16_t* hi
   return __builtin_bit_cast(bf16x8, v);
 }
 
-template <int PI, int PS>
+template <int C, int PI, int PS>
 __global__ __launch_bounds__(512) void k_scan_fwd_quad(GdnArgs A) {
   static_assert(PI != P_F32 && PS != P_F32, "the bf16 modes");
-  constexpr int C = 128, D = 128, DVT = 32, NT = 512;
+  static_assert(C == 64 || C == 128, "half the chunk's rows in whole 32-row steps");
+  constexpr int D = 128, DVT = 32, NT = 512;
+  constexpr int TV = C / 32, SV = C / 64;              // a wave's v_new tiles, their 32-row steps
+  constexpr int NI = C * D / 4 / 256;                  // 4-value slots of a loader thread
   constexpr int PL = C * D;                            // elements of a plane
   constexpr int NW = PS == P_BF16X3 ? 2 : 1, NK = PI == P_BF16X3 ? 2 : 1;  // planes of -w and k
   __shared__ __align__(16) uint16_t sW[NW * PL];       // -w [token][dk], swizzled
@@ -1819,8 +1823,8 @@ __global__ __launch_bounds__(512) void k_scan_fwd_quad(GdnArgs A) {
     const int rh = w >> 1;                  // the wave's 64 rows of both products
     const int col = j0 + 16 * (w & 1);      // its first value column
     const int r = l & 15, g = l >> 4;
-    // A fragments of -w: row 64 rh + 16 t + r, units 4 s + g (swizzled: the row's low bits are r's)
-    const uint16_t* wp = sW + (64 * rh + r) * D;
+    // A fragments of -w: row C/2 rh + 16 t + r, units 4 s + g (swizzled: the row's low bits are r's)
+    const uint16_t* wp = sW + (C / 2 * rh + r) * D;
     const int wu = (g ^ swz(r)) << 3;       // s even; s odd: ^ 32
     // of k^T: dk column 64 rh + 16 t + r, tokens 32 s + 8 g .. + 7
     const uint16_t* kp[2];                  // rows 0-3 and 4-7 of the eight, less the unit
@@ -1833,7 +1837,7 @@ __global__ __launch_bounds__(512) void k_scan_fwd_quad(GdnArgs A) {
       for (int t = 0; t < 4; ++t) ku[e][t] = ((8 * rh + 2 * t + ((r & 3) >> 1)) ^ swz(row)) << 3;
     }
     f32x4 accS[4];  // S[64 rh + 16 t + 4 (lane/16) + rr][col + lane % 16]
-    f32x4 accV[4];  // v_new[64 rh + 16 t + 4 (lane/16) + rr][col + lane % 16]
+    f32x4 accV[TV];  // v_new[C/2 rh + 16 t + 4 (lane/16) + rr][col + lane % 16]
     zero(accS);
     if (n0 == 0 && A.init_state) {
       const float* s0 = A.init_state + (size_t)bh * D * D + col + acc_col();
@@ -1842,24 +1846,24 @@ __global__ __launch_bounds__(512) void k_scan_fwd_quad(GdnArgs A) {
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) accS[t][rr] = s0[(size_t)(64 * rh + 16 * t + acc_row(rr)) * D];
     }
-    float u[4][4];  // u at v_new's layout, loaded a chunk ahead
+    float u[TV][4];  // u at v_new's layout, loaded a chunk ahead
     auto fetch_u = [&](int n) {
       const float* ug = A.uu + hoff(A, b, h, A.H, n, C, D) + col;
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < TV; ++t)
 #pragma unroll
-        for (int rr = 0; rr < 4; ++rr) u[t][rr] = *lane_ptr(ug, 64 * rh + 16 * t + acc_row(rr), D, acc_col());
+        for (int rr = 0; rr < 4; ++rr) u[t][rr] = *lane_ptr(ug, C / 2 * rh + 16 * t + acc_row(rr), D, acc_col());
     };
     // the wave's own two steps of a B operand from its accumulator tiles, to the partner's box
-    auto post = [&](auto& f, const f32x4 (&acc)[4], int bx, const float* scale) {
+    auto post = [&](auto& f, const auto& acc, int bx, const float* scale) {
       constexpr int P = sizeof(f[0]) == sizeof(Frag<P_BF16X3>) ? P_BF16X3 : P_BF16;
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < (int)(sizeof(f) / sizeof(f[0])); ++j) {
         float v[8];
         acc_pair_to_b(acc[2 * j], acc[2 * j + 1], v);
         if (scale) {  // the lane's 8 contraction rows
-          const float4 s0 = *reinterpret_cast<const float4*>(scale + 64 * rh + 32 * j + 8 * g);
-          const float4 s1 = *reinterpret_cast<const float4*>(scale + 64 * rh + 32 * j + 8 * g + 4);
+          const float4 s0 = *reinterpret_cast<const float4*>(scale + C / 2 * rh + 32 * j + 8 * g);
+          const float4 s1 = *reinterpret_cast<const float4*>(scale + C / 2 * rh + 32 * j + 8 * g + 4);
           v[0] *= s0.x; v[1] *= s0.y; v[2] *= s0.z; v[3] *= s0.w;
           v[4] *= s1.x; v[5] *= s1.y; v[6] *= s1.z; v[7] *= s1.w;
         }
@@ -1871,14 +1875,14 @@ __global__ __launch_bounds__(512) void k_scan_fwd_quad(GdnArgs A) {
     auto take = [&](auto& f, int bx) {
       constexpr int P = sizeof(f[0]) == sizeof(Frag<P_BF16X3>) ? P_BF16X3 : P_BF16;
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < (int)(sizeof(f) / sizeof(f[0])); ++j) {
         f[j].hi = __builtin_bit_cast(bf16x8, box[bx][j][0][l]);
         if constexpr (P == P_BF16X3) f[j].lo = __builtin_bit_cast(bf16x8, box[bx][j][1][l]);
       }
     };
-    auto frag_w = [&](Frag<PS> (&fa)[4], int s) {
+    auto frag_w = [&](Frag<PS> (&fa)[TV], int s) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
+      for (int t = 0; t < TV; ++t) {
         const uint16_t* p = wp + 16 * t * D + ((wu ^ (32 * (s & 1))) + 64 * (s >> 1));
         fa[t].hi = *reinterpret_cast<const bf16x8*>(p);
         if constexpr (PS == P_BF16X3) fa[t].lo = *reinterpret_cast<const bf16x8*>(p + PL);
@@ -1895,7 +1899,7 @@ __global__ __launch_bounds__(512) void k_scan_fwd_quad(GdnArgs A) {
     fetch_u(nb);
     for (int n = nb; n < n1; ++n) {
       const bool emit = n >= n0;  // the replayed chunk n0 - 1 only rebuilds the state
-      Frag<PS> own[2], other[2], fw[2][4];
+      Frag<PS> own[2], other[2], fw[2][TV];
       post(own, accS, w ^ 2, nullptr);
       if (emit) {
         StateT<PS>* sg = states_ptr<PS>(A) + ((size_t)bh * A.N + n) * D * D + (size_t)(64 * rh) * D + col;
@@ -1916,7 +1920,7 @@ __global__ __launch_bounds__(512) void k_scan_fwd_quad(GdnArgs A) {
       frag_w(fw[0], 0);
       take(other, w);
 #pragma unroll
-      for (int t = 0; t < 4; ++t) accV[t] = f32x4{u[t][0], u[t][1], u[t][2], u[t][3]};
+      for (int t = 0; t < TV; ++t) accV[t] = f32x4{u[t][0], u[t][1], u[t][2], u[t][3]};
       fetch_u(n + 1 < n1 ? n + 1 : n);
 #pragma unroll
       for (int s = 0; s < 4; ++s) {  // P1: v_new = u + (-w) S
@@ -1924,14 +1928,14 @@ __global__ __launch_bounds__(512) void k_scan_fwd_quad(GdnArgs A) {
         __builtin_amdgcn_sched_barrier(0);
         const Frag<PS> fb = (s >> 1) == rh ? own[s & 1] : other[s & 1];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) mma<PS>(accV[t], fw[s & 1][t], fb);
+        for (int t = 0; t < TV; ++t) mma<PS>(accV[t], fw[s & 1][t], fb);
       }
-      Frag<PI> vown[2], vother[2], fk[2][4];
+      Frag<PI> vown[SV], vother[SV], fk[2][4];
       post(vown, accV, w, skws[n & 1]);
       if (emit) {
-        float* vg = A.vnew + hoff(A, b, h, A.H, n, C, D) + (size_t)(64 * rh) * D + col;
+        float* vg = A.vnew + hoff(A, b, h, A.H, n, C, D) + (size_t)(C / 2 * rh) * D + col;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) st_tile(vg + 16 * t * D, D, accV[t]);
+        for (int t = 0; t < TV; ++t) st_tile(vg + 16 * t * D, D, accV[t]);
       }
       __syncthreads();  // chunk n's k staged, the v_new fragments posted
       frag_k(fk[0], 0);
@@ -1940,10 +1944,10 @@ __global__ __launch_bounds__(512) void k_scan_fwd_quad(GdnArgs A) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) accS[t] *= carry;
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {  // P2: S = carry S + k^T (kws v_new)
-        if (s + 1 < 4) frag_k(fk[(s + 1) & 1], s + 1);
+      for (int s = 0; s < C / 32; ++s) {  // P2: S = carry S + k^T (kws v_new)
+        if (s + 1 < C / 32) frag_k(fk[(s + 1) & 1], s + 1);
         __builtin_amdgcn_sched_barrier(0);
-        const Frag<PI> fb = (s >> 1) == rh ? vown[s & 1] : vother[s & 1];
+        const Frag<PI> fb = s / SV == rh ? vown[s % SV] : vother[s % SV];
 #pragma unroll
         for (int t = 0; t < 4; ++t) mma<PI>(accS[t], fk[s & 1][t], fb);
       }
@@ -1952,7 +1956,7 @@ __global__ __launch_bounds__(512) void k_scan_fwd_quad(GdnArgs A) {
   }
   // ---- loader waves
   const int lt = (int)threadIdx.x - 256;
-  float4 wr[16], kr[16];  // 4096 float4 slots each
+  float4 wr[NI], kr[NI];
   int gs, gsc, gprev;
   float gg, gl, ggc, glc;
   // slot it of a thread: row lt / 32 + 8 it, columns 4 (lt % 32) .. + 3 (the row's swizzle is the
@@ -1960,16 +1964,16 @@ __global__ __launch_bounds__(512) void k_scan_fwd_quad(GdnArgs A) {
   const int row0 = lt >> 5, c4 = lt & 31;
   const unsigned goff = row0 * D + 4 * c4;
   const int soff = swz_at(row0, c4 >> 1) + 4 * (c4 & 1);
-  auto fetch = [&](float4 (&x)[16], const float* src) {
+  auto fetch = [&](float4 (&x)[NI], const float* src) {
 #pragma unroll
-    for (int it = 0; it < 16; ++it) x[it] = *reinterpret_cast<const float4*>(src + 8 * it * D + goff);
+    for (int it = 0; it < NI; ++it) x[it] = *reinterpret_cast<const float4*>(src + 8 * it * D + goff);
   };
   auto fetch_w = [&](int n) { fetch(wr, A.ww + hoff(A, b, h, A.H, n, C, D)); };
   auto fetch_k = [&](int n) { fetch(kr, A.kn + hoff(A, b, hk, A.Hk, n, C, D)); };
   // rows as split planes (sgn: the sign of the staged values)
-  auto put = [&](uint16_t* dst, const float4 (&x)[16], auto planes, float sgn) {
+  auto put = [&](uint16_t* dst, const float4 (&x)[NI], auto planes, float sgn) {
 #pragma unroll
-    for (int it = 0; it < 16; ++it) {
+    for (int it = 0; it < NI; ++it) {
       uint16_t* p = dst + soff + 8 * it * D;
       const float a = sgn * x[it].x, c = sgn * x[it].y, d = sgn * x[it].z, e = sgn * x[it].w;
       if constexpr (decltype(planes)::value == 2) {
