@@ -163,6 +163,8 @@ hipError_t run(const GdnArgs& A, hipStream_t st, int backward, const Timer* tm) 
   const dim3 tiles(chains * parts);
   const int units = A.B * A.H * A.N, cus = cu_count();
   const dim3 persist(units < cus ? units : cus);
+  const int room = wgs_per_cu<C, D, PI>() * cus;
+  const dim3 persist_two(units < room ? units : room);
   auto mark = [&](int k, int end) {
     if (tm) tm->mark(tm->self, k, end, st);
   };
@@ -178,42 +180,42 @@ hipError_t run(const GdnArgs& A, hipStream_t st, int backward, const Timer* tm) 
     if (A.res == 0) {
       if (L.fuse_v) {
         if constexpr (kFV) {
-          if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, true, true>), persist, dim3(C * 4));
-          else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, false, true>), persist, dim3(C * 4));
+          if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, true, true>), persist_two, dim3(C * 4));
+          else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, false, true>), persist_two, dim3(C * 4));
         }
-      } else if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, true>), persist, dim3(C * 4));
-      else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, false>), persist, dim3(C * 4));
+      } else if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, true>), persist_two, dim3(C * 4));
+      else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, false>), persist_two, dim3(C * 4));
     } else {  // T kept for the backward
       if (L.fuse_v) {
         if constexpr (kFV) {
-          if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, true, true>), persist, dim3(C * 4));
-          else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, false, true>), persist, dim3(C * 4));
+          if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, true, true>), persist_two, dim3(C * 4));
+          else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, false, true>), persist_two, dim3(C * 4));
         }
-      } else if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, true>), persist, dim3(C * 4));
-      else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, false>), persist, dim3(C * 4));
+      } else if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, true>), persist_two, dim3(C * 4));
+      else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, false>), persist_two, dim3(C * 4));
     }
     if constexpr (C >= 64 && D == 128 && PI != P_F32) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_quad<C, PI, PS>), tiles, dim3(512));
     else if constexpr (C == 128 && D == 128) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_split<PI, PS>), tiles, dim3(512));
     else GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd<C, D, DVT, PI, PS>), tiles, dim3(NS));
     if (L.fuse_q) {
       if constexpr (kFV) {
-        if (A.ny) GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO, true, true>), persist, dim3(C * 4));
-        else GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO, false, true>), persist, dim3(C * 4));
+        if (A.ny) GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO, true, true>), persist_two, dim3(C * 4));
+        else GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO, false, true>), persist_two, dim3(C * 4));
       }
-    } else if (A.ny) GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO, true>), persist, dim3(C * 4));
-    else GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO>), persist, dim3(C * 4));
+    } else if (A.ny) GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO, true>), persist_two, dim3(C * 4));
+    else GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO>), persist_two, dim3(C * 4));
     if (const unsigned tail = tail_blocks<D, TIO>(A)) GDN_LAUNCH(K_FINAL_STATE, (k_tail<C, D, TIO>), dim3(tail), dim3(256));
   } else {
     const int wouts = A.d_conv_w ? A.taps * A.W : 0;  // one workgroup per head, then the conv weights
     if (A.taps <= 4) GDN_LAUNCH(K_PREP_BWD, (k_prep<C, D, TIO, TG, 3>), prep, dim3(256));
     else GDN_LAUNCH(K_PREP_BWD, (k_prep<C, D, TIO, TG, 4>), prep, dim3(256));
     if (A.res == 0) {  // T and v_new rebuilt
-      if (A.inv == 0) GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 1, true>), persist, dim3(C * 4));
-      else GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 1, false>), persist, dim3(C * 4));
+      if (A.inv == 0) GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 1, true>), persist_two, dim3(C * 4));
+      else GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 1, false>), persist_two, dim3(C * 4));
     } else if (A.res == 1) {  // v_new from the saved T
-      GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 3, false>), persist, dim3(C * 4));
+      GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 3, false>), persist_two, dim3(C * 4));
     }  // else both saved
-    GDN_LAUNCH(K_BWD_LOCAL, (k_bwd_local<C, D, PI, TIO>), persist, dim3(C * 4));
+    GDN_LAUNCH(K_BWD_LOCAL, (k_bwd_local<C, D, PI, TIO>), persist_two, dim3(C * 4));
     GDN_LAUNCH(K_SCAN_BWD, (k_scan_bwd<C, D, DVT, PI, PS, TIO>), tiles, dim3(NS));
     GDN_LAUNCH(K_BWD_GRADS, (k_bwd_grads<C, D, PI, PS, TIO>), chunks, dim3(C * 4));
     // the conv halo sized to the taps (taps - 1 <= 3 for the model's conv of 4); d(conv w)
@@ -248,6 +250,8 @@ hipError_t run_v2(const GdnArgs& A, hipStream_t st, int backward, const Timer* t
   const dim3 tiles(chains * parts);
   const int units = A.B * A.H * A.N, cus = cu_count();
   const dim3 persist(units < cus ? units : cus);
+  const int room = wgs_per_cu<C, D, PI>() * cus;
+  const dim3 persist_two(units < room ? units : room);
   auto mark = [&](int k, int end) {
     if (tm) tm->mark(tm->self, k, end, st);
   };
@@ -260,26 +264,26 @@ hipError_t run_v2(const GdnArgs& A, hipStream_t st, int backward, const Timer* t
   if (!backward) {
     GDN_LAUNCH(K_PREP_FWD, (k_prep_v2<C, D, TIO, TQK, TG>), ends, dim3(256));
     if (A.res == 0) {
-      if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, true>), persist, dim3(C * 4));
-      else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, false>), persist, dim3(C * 4));
+      if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, true>), persist_two, dim3(C * 4));
+      else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, false>), persist_two, dim3(C * 4));
     } else {
-      if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, true>), persist, dim3(C * 4));
-      else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, false>), persist, dim3(C * 4));
+      if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, true>), persist_two, dim3(C * 4));
+      else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, false>), persist_two, dim3(C * 4));
     }
     if constexpr (C >= 64 && D == 128 && PI != P_F32) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_quad<C, PI, PS>), tiles, dim3(512));
     else if constexpr (C == 128 && D == 128) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_split<PI, PS>), tiles, dim3(512));
     else GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd<C, D, DVT, PI, PS>), tiles, dim3(NS));
-    GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO>), persist, dim3(C * 4));
+    GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO>), persist_two, dim3(C * 4));
     if (const unsigned tail = tail_blocks<D, TIO>(A)) GDN_LAUNCH(K_FINAL_STATE, (k_tail<C, D, TIO>), dim3(tail), dim3(256));
   } else {
     GDN_LAUNCH(K_PREP_BWD, (k_prep_v2<C, D, TIO, TQK, TG>), ends, dim3(256));
     if (A.res == 0) {
-      if (A.inv == 0) GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 1, true>), persist, dim3(C * 4));
-      else GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 1, false>), persist, dim3(C * 4));
+      if (A.inv == 0) GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 1, true>), persist_two, dim3(C * 4));
+      else GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 1, false>), persist_two, dim3(C * 4));
     } else if (A.res == 1) {
-      GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 3, false>), persist, dim3(C * 4));
+      GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 3, false>), persist_two, dim3(C * 4));
     }
-    GDN_LAUNCH(K_BWD_LOCAL, (k_bwd_local<C, D, PI, TIO>), persist, dim3(C * 4));
+    GDN_LAUNCH(K_BWD_LOCAL, (k_bwd_local<C, D, PI, TIO>), persist_two, dim3(C * 4));
     GDN_LAUNCH(K_SCAN_BWD, (k_scan_bwd<C, D, DVT, PI, PS, TIO>), tiles, dim3(NS));
     GDN_LAUNCH(K_BWD_GRADS, (k_bwd_grads<C, D, PI, PS, TIO>), chunks_grid(A), dim3(C * 4));
     GDN_LAUNCH(K_POST, (k_post_v2<C, D, TIO, TQK, TG>), ends, dim3(256));

@@ -946,6 +946,19 @@ struct StripA {
       tile_row<P, TN>(acc, fa, B, j0, 32 * s + kg, ok, tn);
     }
   }
+  // product's 32-deep steps [S0, S1) with B holding the contraction from 32 S0 on
+  template <int P, int S0, int S1, int TN, class BV>
+  __device__ __forceinline__ void product_steps(f32x4 (&acc)[TN], const BV& B, float rs) const {
+    static_assert(K % 32 == 0, "whole steps");
+    const int kg = (lane() >> 4) << 3;
+#pragma unroll
+    for (int s = S0; s < S1; ++s) {
+      float xs[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xs[e] = x[s][e] * rs;
+      tile_row<P, TN>(acc, make_frag<a_prec<P>()>(xs), B, 0, 32 * (s - S0) + kg, true, TN);
+    }
+  }
   // the transposed product: acc[t] += B(i0 + 16t .., .) (strip)^T for the tiles t < TM, B a view
   // or operand tile whose rows are the M index (the strip is the B operand, its rows the N index)
   template <int P, int TM, class AV>
@@ -1000,6 +1013,21 @@ struct StripIO {
       for (int e = 0; e < 8; ++e) xs[e] = ok ? xs[e] * f : 0.f;
       const Frag<a_prec<P>()> fa = make_frag<a_prec<P>()>(xs);
       tile_row<P, TN>(acc, fa, B, j0, 32 * s + kg, ok, tn);
+    }
+  }
+  // product's 32-deep steps [S0, S1) with B holding the contraction from 32 S0 on
+  template <int P, int S0, int S1, int TN, class BV>
+  __device__ __forceinline__ void product_steps(f32x4 (&acc)[TN], const BV& B, float rs) const {
+    static_assert(K % 32 == 0, "whole steps");
+    const int kg = (lane() >> 4) << 3;
+    const float f = valid ? rs : 0.f;
+#pragma unroll
+    for (int s = S0; s < S1; ++s) {
+      float xs[8];
+      x[s].get(xs);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xs[e] *= f;
+      tile_row<P, TN>(acc, make_frag<a_prec<P>()>(xs), B, 0, 32 * (s - S0) + kg, true, TN);
     }
   }
 };
@@ -1143,6 +1171,18 @@ struct RawV {
   }
 };
 
+// ---------------------------------------------------------------- workgroups per CU
+// A chunk kernel's workgroup is one wave per 16 token rows: 4 waves at a chunk of 64, one per
+// SIMD, and its phases (staging, barriers, products) leave the SIMD idle most of the time. At D =
+// 128 in the bf16 modes those kernels keep to half the CU's LDS and registers (operand regions of
+// the operands' own shapes, D x D states staged in two halves) and two workgroups run per CU.
+// Measured at two rows of 1777 tokens, 32 heads (1792 units): k_chunk 89 -> 64 us forward, 107 -> 94
+// backward, k_out 109 -> 79, k_bwd_local 96 -> 66, k_bwd_grads 182 -> 156. (Eight waves per
+// workgroup, two per strip, instead: k_chunk 84 with one workgroup per CU, 83 with two, at 128
+// registers.) At a chunk of 128 the operands alone pass half the LDS.
+template <int C, int D, int PI>
+constexpr int wgs_per_cu() { return C == 64 && D == 128 && PI != P_F32 ? 2 : 1; }
+
 // ---------------------------------------------------------------- k_chunk
 // Persistent over the (row, head, chunk) units as k_out; C/16 waves (one 16-row strip each).
 // MODE 0 (forward): writes w and u; MODE 2: also T (kept as a residual). MODE 1 (backward
@@ -1156,15 +1196,19 @@ struct RawV {
 // a template argument: both forms in one kernel take 17 more VGPRs and spill in MODE 1). FV: the
 // forward's v built from the raw rows (RawV) instead of read from k_prep's rows.
 template <int C, int D, int PI, int PS, int MODE, bool DBL, bool FV = false>
-__global__ __launch_bounds__(C * 4) void k_chunk(GdnArgs A) {
+__global__ __launch_bounds__(C * 4, (wgs_per_cu<C, D, PI>())) void k_chunk(GdnArgs A) {
   constexpr bool FWD = MODE == 0 || MODE == 2;  // writes w and u (else v_new)
   constexpr bool LOAD_T = MODE == 3;            // T from the residuals
   constexpr bool STORE_T = MODE == 1 || MODE == 2;
   constexpr int NT = C * 4;
-  constexpr int M = C > D ? C : D;
-  constexpr int LT = M + 4;
-  using TB = OpTile<PI, M, M>;
-  constexpr int RB = TB::BYTES > C * LT * 4 ? TB::BYTES : C * LT * 4;  // also T^T during the inverse
+  constexpr int LT = C + 4;
+  constexpr int NH = wgs_per_cu<C, D, PI>();  // S is staged in NH parts of its dk rows
+  using TR = OpTile<PI, C, D>;                // k rows
+  using TK = OpTile<PI, D, C>;                // kbe^T, (v beta)^T, Y^T
+  using TS = OpTile<PI, D, D / NH>;           // S^T, of one part
+  constexpr int RK = TR::BYTES > TK::BYTES ? TR::BYTES : TK::BYTES;
+  constexpr int RS = FWD || TS::BYTES < RK ? RK : TS::BYTES;
+  constexpr int RB = RS > C * LT * 4 ? RS : C * LT * 4;  // also T^T during the inverse
   __shared__ __align__(16) float sT[C * LT];
   __shared__ __align__(16) char sB[RB];
   __shared__ Ctx<C> cx;
@@ -1172,7 +1216,7 @@ __global__ __launch_bounds__(C * 4) void k_chunk(GdnArgs A) {
   static_assert(!FV || FWD, "FV: the forward modes");
   GDN_POISON_LDS(sT, sB, cx, sW);
   const int w = wave(), i0 = 16 * w;
-  const Op<PI> ob = TB::at(sB);
+  const Op<PI> orow = TR::at(sB), ob = TK::at(sB), os = TS::at(sB);
   const int total = A.B * A.H * A.N;
   CtxRaw<C, FV> rc;
   RegsT<C, D, NT> kk;  // k: staged as rows (A and B of k k^T), then as kbe^T
@@ -1187,10 +1231,10 @@ __global__ __launch_bounds__(C * 4) void k_chunk(GdnArgs A) {
     const size_t off = hoff(A, x.b, x.h, A.H, x.n, C, D);
     TinvT<PI>* tg = tinv_ptr<PI>(A) + ((size_t)(x.b * A.H + x.h) * A.N + x.n) * C * C;
     rc.commit(cx);
-    if constexpr (!LOAD_T) kk.put_rows(ob);
+    if constexpr (!LOAD_T) kk.put_rows(orow);
     rc.fetch(A, y.b, y.h, y.n);
     std::conditional_t<FV, RawV<C, D, NT>, RegsT<C, D, NT>> vc;  // this unit's (v beta)^T source (forward)
-    RegsT<D, D, NT, true, StateT<PS>> sc;  // S_before, its strip of k and its v at the accumulator layout (backward)
+    RegsT<D / NH, D, NT, true, StateT<PS>> sc;  // S_before (one part), its strip of k and its v at the accumulator layout (backward)
     StripA<D> ks;
     AccVals<D / 16> va;
     if constexpr (LOAD_T) {
@@ -1206,7 +1250,7 @@ __global__ __launch_bounds__(C * 4) void k_chunk(GdnArgs A) {
       {  // L = strict(beta_i (k k^T)_ij D_ij): tiles on and below the diagonal only
         f32x4 acc[C / 16];
         zero(acc);
-        strip_mma<PI, D, C / 16>(acc, ob, i0, ob, 0, 0, D, w + 1);
+        strip_mma<PI, D, C / 16>(acc, orow, i0, orow, 0, 0, D, w + 1);
         // every tile's values first, then the stores: the single stores' memory clobber would
         // otherwise keep the next tile's context reads (LDS) behind them
         const StripDecay<C> sd(cx, i0);
@@ -1244,9 +1288,19 @@ __global__ __launch_bounds__(C * 4) void k_chunk(GdnArgs A) {
     if constexpr (!FWD) {  // v_new = T (v beta - kbe S_before): one state-path product, one with T
       f32x4 yv[D / 16];
       zero(yv);
-      sc.put_cols(ob);  // S^T
-      __syncthreads();
-      ks.template product<PS>(yv, ob, 0, D / 16, -cx.bg[i0 + (lane() & 15)]);  // - kbe S
+      sc.put_cols(os);  // S^T
+      if constexpr (NH == 1) {
+        __syncthreads();
+        ks.template product<PS>(yv, os, 0, D / 16, -cx.bg[i0 + (lane() & 15)]);  // - kbe S
+      } else {
+        sc.fetch(states_ptr<PS>(A) + ((size_t)(x.b * A.H + x.h) * A.N + x.n) * D * D + D / 2 * D, D);
+        __syncthreads();
+        ks.template product_steps<PS, 0, D / 64>(yv, os, -cx.bg[i0 + (lane() & 15)]);
+        __syncthreads();
+        sc.put_cols(os);
+        __syncthreads();
+        ks.template product_steps<PS, D / 64, D / 32>(yv, os, -cx.bg[i0 + (lane() & 15)]);
+      }
 #pragma unroll
       for (int t = 0; t < D / 16; ++t)
 #pragma unroll
@@ -2125,23 +2179,26 @@ struct RawQ {
 // k_prep's rows. Every global input of a unit is held in registers and refilled
 // with the next unit's values right after it has been used, so its loads run during the rest
 // of the unit instead of stalling the next one.
-template <int C, int D, int NT, class TS, bool FQ = false>
+template <int C, int D, int NT, class TS, bool FQ = false, int NH = 1>
 struct OutIn {
   CtxRaw<C, FQ> cx;
   Regs<C, D, NT> k;      // k rows: B(d, j) = k[j][d]
   std::conditional_t<FQ, RawQ<C, D>, StripA<D>> q;  // this wave's q rows (A operand of q k^T and of q_read S)
   RegsT<C, D, NT> v;     // v_new rows, staged as v_new^T
-  RegsT<D, D, NT, true, TS> st;  // S_before rows, staged as S^T
+  RegsT<D / NH, D, NT, true, TS> st;  // S_before rows (one of NH parts), staged as S^T
 };
 
 template <int C, int D, int PI, int PS, class TIO, bool NORM = false, bool FQ = false>
-__global__ __launch_bounds__(C * 4) void k_out(GdnArgs A) {
+__global__ __launch_bounds__(C * 4, (wgs_per_cu<C, D, PI>())) void k_out(GdnArgs A) {
   constexpr int NT = C * 4;
   constexpr int LI = C + 4;
-  constexpr int M = C > D ? C : D;
-  using TB = OpTile<PI, M, M>;
+  constexpr int NH = wgs_per_cu<C, D, PI>();  // S is staged in NH parts of its dk rows
+  using TR = OpTile<PI, C, D>;                // k rows
+  using TK = OpTile<PI, D, C>;                // v_new^T
+  using TS = OpTile<PI, D, D / NH>;           // S^T, of one part
+  constexpr int RK = TR::BYTES > TK::BYTES ? TR::BYTES : TK::BYTES;
   __shared__ __align__(16) float sI[C * LI];  // also the staged raw q rows (FQ)
-  __shared__ __align__(16) char sB[TB::BYTES];
+  __shared__ __align__(16) char sB[TS::BYTES > RK ? TS::BYTES : RK];
   __shared__ Ctx<C> cx;
   __shared__ __align__(16) float snw[NORM ? D : 1];  // the norm's weight
   __shared__ __align__(16) float sWq[FQ ? 4 * D : 4];  // FQ: the unit's conv weights of q
@@ -2150,18 +2207,20 @@ __global__ __launch_bounds__(C * 4) void k_out(GdnArgs A) {
   if constexpr (NORM) {
     for (int c = threadIdx.x; c < D; c += NT) snw[c] = A.nw[c];
   }
-  const Op<PI> ob = TB::at(sB);
+  const Op<PI> orow = TR::at(sB), ob = TK::at(sB), os = TS::at(sB);
   const int ws = wave_strip<C / 16, false>();
   const int total = A.B * A.H * A.N;
-  OutIn<C, D, NT, StateT<PS>, FQ> in;
+  OutIn<C, D, NT, StateT<PS>, FQ, NH> in;
   {
     const UnitIx<BY_HEAD> x(A, blockIdx.x);
     in.cx.fetch(A, x.b, x.h, x.n);
     in.k.fetch(A.kn + hoff(A, x.b, x.hk, A.Hk, x.n, C, D), D);
     if constexpr (FQ) in.q.fetch(A, x.b, x.hk, x.n, 16 * ws);
     else in.q.fetch(A.qn + hoff(A, x.b, x.hk, A.Hk, x.n, C, D), D, 16 * ws);
-    in.v.fetch(A.vnew + hoff(A, x.b, x.h, A.H, x.n, C, D), D);
-    in.st.fetch(states_ptr<PS>(A) + ((size_t)x.b * A.H + x.h) * A.N * D * D + (size_t)x.n * D * D, D);
+    if constexpr (NH == 1) {
+      in.v.fetch(A.vnew + hoff(A, x.b, x.h, A.H, x.n, C, D), D);
+      in.st.fetch(states_ptr<PS>(A) + ((size_t)x.b * A.H + x.h) * A.N * D * D + (size_t)x.n * D * D, D);
+    }
   }
   for (int u = blockIdx.x; u < total; u += gridDim.x) {
     const int w = opaque_uniform(ws), i0 = 16 * w;  // conditions on w stay in the loop
@@ -2169,7 +2228,9 @@ __global__ __launch_bounds__(C * 4) void k_out(GdnArgs A) {
     const UnitIx<BY_HEAD> y(A, u + gridDim.x < total ? u + gridDim.x : u);  // the next unit (or this one again)
     in.cx.commit(cx);
     in.cx.fetch(A, y.b, y.h, y.n);
-    in.k.put_rows(ob);
+    in.k.put_rows(orow);
+    // two workgroups per CU: v_new and S come a stage ahead, not a unit ahead (registers)
+    if constexpr (NH > 1) in.v.fetch(A.vnew + hoff(A, x.b, x.h, A.H, x.n, C, D), D);
     if constexpr (FQ) in.q.stage(reinterpret_cast<char*>(sI), sWq, A, i0);
     __syncthreads();
     derive_ctx<C, NT>(cx);
@@ -2180,7 +2241,7 @@ __global__ __launch_bounds__(C * 4) void k_out(GdnArgs A) {
     {
       f32x4 acc[C / 16];
       zero(acc);
-      qs.template product<PI>(acc, ob, 0, w + 1);
+      qs.template product<PI>(acc, orow, 0, w + 1);
       // refills are issued after the product that follows each staging: the staged
       // registers are then not live across that product
       in.k.fetch(A.kn + hoff(A, y.b, y.hk, A.Hk, y.n, C, D), D);
@@ -2195,13 +2256,15 @@ __global__ __launch_bounds__(C * 4) void k_out(GdnArgs A) {
     }
     __syncthreads();
     in.v.put_cols(ob);
+    if constexpr (NH > 1)
+      in.st.fetch(states_ptr<PS>(A) + ((size_t)x.b * A.H + x.h) * A.N * D * D + (size_t)x.n * D * D, D);
     __syncthreads();
     f32x4 o[D / 16];
     zero(o);
     strip_mma<PI, C, D / 16>(o, krow(sI, LI), i0, ob, 0, 0, tri_end<C>(i0));
-    in.v.fetch(A.vnew + hoff(A, y.b, y.h, A.H, y.n, C, D), D);
+    if constexpr (NH == 1) in.v.fetch(A.vnew + hoff(A, y.b, y.h, A.H, y.n, C, D), D);
     __syncthreads();
-    in.st.put_cols(ob);
+    in.st.put_cols(os);
     // the lane's output row after the quad transposes below (4 consecutive columns per tile)
     const int tok = x.n * C + i0 + ((lane() >> 4) << 2) + (lane() & 3);
     const size_t orow = (((size_t)x.b * A.T + (tok < A.T ? tok : 0)) * A.H + x.h) * D + (lane() & 12);
@@ -2210,11 +2273,22 @@ __global__ __launch_bounds__(C * 4) void k_out(GdnArgs A) {
 #pragma unroll
       for (int t = 0; t < D / 16; ++t) zr[t].load(reinterpret_cast<const TIO*>(A.nz) + orow + 16 * t);
     }
-    __syncthreads();
-    qs.template product<PS>(o, ob, 0, D / 16, cx.grow[i0 + (lane() & 15)]);
+    if constexpr (NH == 1) {
+      __syncthreads();
+      qs.template product<PS>(o, os, 0, D / 16, cx.grow[i0 + (lane() & 15)]);
+    } else {
+      in.st.fetch(states_ptr<PS>(A) + ((size_t)x.b * A.H + x.h) * A.N * D * D + (size_t)x.n * D * D + D / 2 * D, D);
+      __syncthreads();
+      qs.template product_steps<PS, 0, D / 64>(o, os, cx.grow[i0 + (lane() & 15)]);
+      __syncthreads();
+      in.st.put_cols(os);
+      __syncthreads();
+      qs.template product_steps<PS, D / 64, D / 32>(o, os, cx.grow[i0 + (lane() & 15)]);
+    }
     if constexpr (FQ) in.q.fetch(A, y.b, y.hk, y.n, i0);
     else in.q.fetch(A.qn + hoff(A, y.b, y.hk, A.Hk, y.n, C, D), D, i0);
-    in.st.fetch(states_ptr<PS>(A) + ((size_t)y.b * A.H + y.h) * A.N * D * D + (size_t)y.n * D * D, D);
+    if constexpr (NH == 1)
+      in.st.fetch(states_ptr<PS>(A) + ((size_t)y.b * A.H + y.h) * A.N * D * D + (size_t)y.n * D * D, D);
     TIO* out = reinterpret_cast<TIO*>(A.out);
     {  // quad transposes: each lane stores 4 consecutive columns of one row
       float ss = 0.f;
@@ -2416,16 +2490,16 @@ struct LocalIn {
 };
 
 template <int C, int D, int PI, class TIO>
-__global__ __launch_bounds__(C * 4) void k_bwd_local(GdnArgs A) {
+__global__ __launch_bounds__(C * 4, (wgs_per_cu<C, D, PI>())) void k_bwd_local(GdnArgs A) {
   constexpr int NT = C * 4;
   constexpr int LA = C + 4;
-  constexpr int M = C > D ? C : D;
-  using TB = OpTile<PI, M, M>;
+  using TR = OpTile<PI, C, D>;  // k rows
+  using TK = OpTile<PI, D, C>;  // do^T, dv_loc^T, k_write^T
   __shared__ float sA[C * LA];
-  __shared__ __align__(16) char sB[TB::BYTES];
+  __shared__ __align__(16) char sB[TR::BYTES > TK::BYTES ? TR::BYTES : TK::BYTES];
   __shared__ Ctx<C> cx;
   GDN_POISON_LDS(sA, sB, cx);
-  const Op<PI> ob = TB::at(sB);
+  const Op<PI> orow = TR::at(sB), ob = TK::at(sB);
   const int ws = wave_strip<C / 16, true>();
   const int total = A.B * A.H * A.N;
   LocalIn<C, D, NT, TIO, TinvT<PI>> in;
@@ -2442,14 +2516,14 @@ __global__ __launch_bounds__(C * 4) void k_bwd_local(GdnArgs A) {
     in.cx.commit(cx);
     in.cx.fetch(A, y.b, y.h, y.n);
     in.fetch_do(A, x);
-    in.k.put_rows(ob);  // B(d, j) = k[j][d]
+    in.k.put_rows(orow);  // B(d, j) = k[j][d]
     __syncthreads();
     derive_ctx<C, NT>(cx);
     __syncthreads();
     {  // intra = (q k^T) . D
       f32x4 acc[C / 16];
       zero(acc);
-      in.q.template product<PI>(acc, ob, 0, w + 1);
+      in.q.template product<PI>(acc, orow, 0, w + 1);
       in.fetch_q(A, y, i0);
       // q k^T on and below the diagonal, for the decay gradient's pair sums: tile (w, t) as 256
       // floats in accumulator order, one 16-byte piece per lane
@@ -2696,20 +2770,23 @@ __global__ __launch_bounds__((C > D ? C : D) * 4) void k_scan_bwd(GdnArgs A) {
 // k^T, q^T through one LDS operand region; m1, then m2, in fp32 LDS (read by rows and by
 // columns); the per-token sums through LDS.
 template <int C, int D, int PI, int PS, class TIO>
-__global__ __launch_bounds__(C * 4) void k_bwd_grads(GdnArgs A) {
+__global__ __launch_bounds__(C * 4, (wgs_per_cu<C, D, PI>())) void k_bwd_grads(GdnArgs A) {
   constexpr int NT = C * 4;
   constexpr int LA = C + 4;
-  constexpr int M = C > D ? C : D;
+  constexpr int NH = wgs_per_cu<C, D, PI>();  // S and G are staged in NH parts of their columns
   constexpr int TD = D / 16;
   constexpr int TC = C / 16;
-  using TB = OpTile<PI, M, M>;
+  using TR = OpTile<PI, C, D>;       // v_new rows
+  using TK = OpTile<PI, D, C>;       // k^T, q^T
+  using TS = OpTile<PI, D, D / NH>;  // S, G: one part
+  constexpr int RK = TR::BYTES > TK::BYTES ? TR::BYTES : TK::BYTES;
   __shared__ float sA[C * LA];
-  __shared__ __align__(16) char sB[TB::BYTES];
+  __shared__ __align__(16) char sB[TS::BYTES > RK ? TS::BYTES : RK];
   __shared__ Ctx<C> cx;
   __shared__ float sga[C], sgf[C], sgb[C];  // a, f and d beta per token
   __shared__ float sxc[TC * C];             // per wave: its rows' share of x_t for the tokens t of its tiles
   GDN_POISON_LDS(sA, sB, cx, sga, sgf, sgb, sxc);
-  const Op<PI> ob = TB::at(sB);
+  const Op<PI> orow = TR::at(sB), ob = TK::at(sB), os = TS::at(sB);
   const int id = blockIdx.x;
   const int n = id % A.N, bh = id / A.N, h = bh % A.H, b = bh / A.H, hk = h / A.ratio;
   const int w = wave_strip<C / 16, true>(), i0 = 16 * w, r = lane() & 15;
@@ -2722,23 +2799,37 @@ __global__ __launch_bounds__(C * 4) void k_bwd_grads(GdnArgs A) {
   xs.fetch(A.xl + off, D, i0);
   dos.fetch(dout + (((size_t)b * A.T + (size_t)n * C) * A.H + h) * D, A.H * D, i0, A.T - n * C);
   load_ctx<C, NT>(cx, A, b, h, n);
-  stage_rows<D, D, NT>(ob, states_ptr<PS>(A) + ((size_t)bh * A.N + n) * D * D, D);  // S: B(dv, j=dk) = S[dk][dv]
-  vn.fetch(A.vnew + off, D, i0);
+  const StateT<PS>* sg = states_ptr<PS>(A) + ((size_t)bh * A.N + n) * D * D;
+  stage_rows<D, D / NH, NT>(os, sg, D);  // S: B(dv, j=dk) = S[dk][dv]
+  if constexpr (NH == 1) vn.fetch(A.vnew + off, D, i0);
   __syncthreads();
   f32x4 dkb[TD], dq[TD];
   zero(dkb);
   zero(dq);
-  xs.template product<PS>(dkb, ob, 0, TD, -cx.grow[i0 + r]);  // -(grow X) S^T
-  dos.template product<PS>(dq, ob, 0, TD, cx.grow[i0 + r]);   // (grow do) S^T
+  if constexpr (NH == 1) {
+    xs.template product<PS>(dkb, os, 0, TD, -cx.grow[i0 + r]);  // -(grow X) S^T
+    dos.template product<PS>(dq, os, 0, TD, cx.grow[i0 + r]);   // (grow do) S^T
+  } else {
+    Regs<D, D / 2, NT, StateT<PS>> s1;
+    s1.fetch(sg + D / 2, D);
+    xs.template product_steps<PS, 0, D / 64>(dkb, os, -cx.grow[i0 + r]);
+    dos.template product_steps<PS, 0, D / 64>(dq, os, cx.grow[i0 + r]);
+    __syncthreads();
+    s1.put_rows(os);
+    vn.fetch(A.vnew + off, D, i0);
+    __syncthreads();
+    xs.template product_steps<PS, D / 64, D / 32>(dkb, os, -cx.grow[i0 + r]);
+    dos.template product_steps<PS, D / 64, D / 32>(dq, os, cx.grow[i0 + r]);
+  }
   __syncthreads();
-  vn.put_rows(ob, i0);  // v_new: B(dv, j) = v_new[j][dv]
+  vn.put_rows(orow, i0);  // v_new: B(dv, j) = v_new[j][dv]
   __syncthreads();
   f32x4 m2[TC];
   {  // m1 -> LDS, m2 -> registers
     f32x4 acc[TC];
     zero(acc);
     const StripDecay<C> sd(cx, i0);
-    xs.template product<PI>(acc, ob, 0, w + 1);
+    xs.template product<PI>(acc, orow, 0, w + 1);
     float dn[4];  // the next tile's decays, read before this tile's stores (their memory clobber)
     sd.tile(cx, i0, 0, w, dn);
 #pragma unroll
@@ -2764,7 +2855,7 @@ __global__ __launch_bounds__(C * 4) void k_bwd_grads(GdnArgs A) {
       }
     }
     zero(m2);
-    dos.template product<exact_a<PI, sizeof(TIO) == 2>()>(m2, ob, 0, w + 1);  // do: bf16 exact
+    dos.template product<exact_a<PI, sizeof(TIO) == 2>()>(m2, orow, 0, w + 1);  // do: bf16 exact
     float rp[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < TC; ++t) {
@@ -2783,11 +2874,22 @@ __global__ __launch_bounds__(C * 4) void k_bwd_grads(GdnArgs A) {
     }
   }
   __syncthreads();
-  stage_rows<D, D, NT>(ob, A.gg + ((size_t)bh * A.N + n) * D * D, D);  // G
+  const float* ggp = A.gg + ((size_t)bh * A.N + n) * D * D;
+  stage_rows<D, D / NH, NT>(os, ggp, D);  // G
   __syncthreads();
   f32x4 dk[TD];
   zero(dk);
-  vn.template product<PS>(dk, ob, 0, TD, cx.kws[i0 + r]);  // (kws v_new) G^T
+  if constexpr (NH == 1) {
+    vn.template product<PS>(dk, os, 0, TD, cx.kws[i0 + r]);  // (kws v_new) G^T
+  } else {
+    Regs<D, D / 2, NT> g1;
+    g1.fetch(ggp + D / 2, D);
+    vn.template product_steps<PS, 0, D / 64>(dk, os, cx.kws[i0 + r]);
+    __syncthreads();
+    g1.put_rows(os);
+    __syncthreads();
+    vn.template product_steps<PS, D / 64, D / 32>(dk, os, cx.kws[i0 + r]);
+  }
   AccVals<TD> kk;  // (k and q are fetched late: live across the stages before, they would spill)
   kk.fetch(kg, D, i0);
   __syncthreads();
