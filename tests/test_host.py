@@ -614,3 +614,14 @@ def test_integration_python_samples_compile():
     assert len(blocks) >= 2
     for i, src in enumerate(blocks):
         compile(src, f"INTEGRATION.md python block {i}", "exec")
+
+
+def test_every_forward_scan_and_tail_symbol_has_a_name():
+    """The profile tables name each kernel by what it does, whichever form ran."""
+    from tjev_amd.profiling import _Namer
+
+    name = _Namer()
+    for form in ("k_scan_fwd<64, 64, 32, 1, 1>", "k_scan_fwd_split<0, 0>", "k_scan_fwd_quad<128, 1, 1>"):
+        assert name(f"void gdn::{form}(gdn::GdnArgs)") == "gdn_scan_fwd"
+    assert name("void gdn::k_tail<128, 128, unsigned short>(gdn::GdnArgs)") == "gdn_final_state"
+    assert name("void gdn::(anonymous namespace)::k_lora_merge<2>(gdn::MergeArgs)") == "gdn_lora_merge"
