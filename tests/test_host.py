@@ -625,3 +625,11 @@ def test_every_forward_scan_and_tail_symbol_has_a_name():
         assert name(f"void gdn::{form}(gdn::GdnArgs)") == "gdn_scan_fwd"
     assert name("void gdn::k_tail<128, 128, unsigned short>(gdn::GdnArgs)") == "gdn_final_state"
     assert name("void gdn::(anonymous namespace)::k_lora_merge<2>(gdn::MergeArgs)") == "gdn_lora_merge"
+
+
+def test_no_stream_of_a_cpu_device():
+    """A raw launch on CPU tensors is refused before any address reaches the library."""
+    from tjev_amd import _lib
+
+    with pytest.raises(ValueError):
+        _lib.current_stream(torch.device("cpu"))
