@@ -46,3 +46,16 @@ def test_merge_refuses_what_it_does_not_hold():
         assert lib.tjev_gdn_lora_merge((_lib.Merge * 1)(_lib.Merge(**{**ok, **bad})), 1, None) == status, bad
     assert lib.tjev_gdn_lora_merge((_lib.Merge * 9)(*[_lib.Merge(**ok)] * 9), 9, None) == 1
     assert lib.tjev_gdn_lora_merge(None, 1, None) == 1
+
+
+@pytest.mark.parametrize("inputs,outputs", [(0, 64), (64, 0), (64, 12)])
+def test_merge_of_other_forms_takes_the_gemm(inputs, outputs):
+    """What the kernel does not hold (no rows, no columns, columns not in multiples of 8) merges as before."""
+    from tjev_amd.block import _merge, _merge_all
+
+    gen = torch.Generator().manual_seed(3)
+    w = torch.randn(inputs, outputs, generator=gen).to(torch.bfloat16).cuda()
+    a, b = torch.randn(inputs, 64, generator=gen).cuda(), torch.randn(64, outputs, generator=gen).cuda()
+    print(f"merge {inputs} x {outputs}", flush=True)
+    (got,) = _merge_all([w], [a], [b], [0.5], torch.bfloat16)
+    assert got.shape == w.shape and torch.equal(got, _merge(w, a, b, 0.5, torch.bfloat16))

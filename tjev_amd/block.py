@@ -71,15 +71,17 @@ def _merge(w: torch.Tensor, a: torch.Tensor, b: torch.Tensor, s: float, dtype) -
 def _merge_all(ws, a_s, b_s, scales, dtype) -> list[torch.Tensor]:
     """``_merge`` of every projection of a group: one launch of the HIP library's merge kernel for bf16
     weights and fp32 adapters of one rank of 32, 64, 96 or 128 (any number of inputs; outputs in
-    multiples of 8), contiguous and 16-byte aligned as parameters are; else one GEMM each. A GEMM
-    with W as its addend first copies W into its output and takes bf16 copies of both adapters:
+    multiples of 8, none empty), contiguous and 16-byte aligned as parameters are; else, and where
+    the call is traced (no addresses to pass), one GEMM each. A GEMM with W as its addend first copies W into its output and takes bf16 copies of both adapters:
     168 us for the 4B layer's five projections against 51 (two launches)."""
     rank = a_s[0].shape[1]
     if (dtype == torch.bfloat16 and len(ws) <= _lib.MAX_MERGE and rank in (32, 64, 96, 128)
+            and not torch.compiler.is_compiling()
             and all(w.is_cuda and w.dtype == dtype and a.dtype == b.dtype == torch.float32 and w.shape[1] % 8 == 0
-                    and a.device == b.device == w.device == ws[0].device
+                    and w.numel() > 0 and a.device == b.device == w.device == ws[0].device
                     and a.shape == (w.shape[0], rank) and b.shape == (rank, w.shape[1])
-                    and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (w, a, b))
+                    and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_contiguous() and t.data_ptr() % 16 == 0
+                            for t in (w, a, b))
                     for w, a, b in zip(ws, a_s, b_s))):
         outs = [torch.empty_like(w) for w in ws]
         args = (_lib.Merge * len(ws))(*(
