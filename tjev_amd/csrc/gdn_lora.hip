@@ -5,12 +5,12 @@
 // Bound by memory: W is read and W' written once in bf16 (2560 x 8192: 84 MB), the adapters are
 // small. A workgroup of 4 waves owns 128 columns and 128 rows: B's columns are rounded into LDS
 // once ([column][rank], so a fragment is one 16-byte read), each wave then takes two strips of 16
-// rows, the second's inputs loaded while the first is computed. The product is accumulated transposed (B^T's fragment as the MFMA's first operand), with
-// the columns of a pair of tiles interleaved so that a lane holds 8 consecutive columns of its
-// row: W and W' move as 16-byte pieces, 64 contiguous bytes per row and instruction. Measured at
-// the 4B layer (qkv, z, b and a of 2560 inputs, rank 64, in one launch): 37 us, 3.4 TB/s,
-// against 134 us for the four GEMMs with their copies; out_proj (4096 x 2560) 14 us against 34; 256 rows
-// per workgroup 37 and 16 us.
+// rows, the second's inputs loaded while the first is computed. The product is accumulated
+// transposed (B^T's fragment as the MFMA's first operand), with the columns of a pair of tiles
+// interleaved so that a lane holds 8 consecutive columns of its row: W and W' move as 16-byte
+// pieces, 64 contiguous bytes per row and instruction. Measured at the 4B layer (qkv, z, b and a
+// of 2560 inputs, rank 64, in one launch): 37 us, 3.4 TB/s, against 134 us for the four GEMMs
+// with their copies; out_proj (4096 x 2560) 14 us against 34; 256 rows per workgroup 37 and 16 us.
 #include <hip/hip_runtime.h>
 
 #include <string>
