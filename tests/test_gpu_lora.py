@@ -59,3 +59,24 @@ def test_merge_of_other_forms_takes_the_gemm(inputs, outputs):
     print(f"merge {inputs} x {outputs}", flush=True)
     (got,) = _merge_all([w], [a], [b], [0.5], torch.bfloat16)
     assert got.shape == w.shape and torch.equal(got, _merge(w, a, b, 0.5, torch.bfloat16))
+
+
+@pytest.mark.parametrize("pre_dispatch", [False, True])
+def test_recorded_merge_stays_in_the_graph(pre_dispatch):
+    """A graph of the projections recorded by make_fx holds the merge as an operator (the kernel's launch is
+    none: its output would be recorded as uninitialised memory) and replays to the same values."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    from tjev_amd.block import LoRALinear, grouped
+
+    gen = torch.Generator().manual_seed(4)
+    w = torch.randn(256, 128, generator=gen).to(torch.bfloat16).cuda()
+    a, b = torch.randn(256, 32, generator=gen).cuda(), torch.randn(32, 128, generator=gen).cuda()
+    x = torch.randn(64, 256, generator=gen).to(torch.bfloat16).cuda()
+    linear = LoRALinear(w, a, b, 0.5)
+    print(f"recorded merge, pre_dispatch={pre_dispatch}", flush=True)
+    want = grouped(x, linear)[0]
+    graph = make_fx(lambda t: grouped(t, linear)[0], pre_dispatch=pre_dispatch)(x)
+    names = [str(n.target) for n in graph.graph.nodes if n.op == "call_function"]
+    assert any("addmm" in n for n in names) and not any("empty" in n for n in names), names
+    assert torch.equal(graph(x), want)

@@ -20,6 +20,8 @@ from __future__ import annotations
 import math
 
 import torch
+from torch._ops import _len_torch_dispatch_stack_pre_dispatch
+from torch.utils._python_dispatch import _get_current_dispatch_mode
 
 from . import _lib
 from .gdn import gdn_megakernel_normed
@@ -68,15 +70,24 @@ def _merge(w: torch.Tensor, a: torch.Tensor, b: torch.Tensor, s: float, dtype) -
     return (w.to(torch.float32) + s * _mm32(a, b)).to(dtype)
 
 
+def _recorded() -> bool:
+    """Whether the operators called here are recorded or replaced rather than only run (torch.compile,
+    jit tracing, a dispatch mode such as make_fx's or a FLOP counter's): a launch by address is
+    no operator, and a recorded graph would hold its output uninitialised."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or _get_current_dispatch_mode() is not None
+            or _len_torch_dispatch_stack_pre_dispatch() > 0)
+
+
 def _merge_all(ws, a_s, b_s, scales, dtype) -> list[torch.Tensor]:
     """``_merge`` of every projection of a group: one launch of the HIP library's merge kernel for bf16
     weights and fp32 adapters of one rank of 32, 64, 96 or 128 (any number of inputs; outputs in
     multiples of 8, none empty), contiguous and 16-byte aligned as parameters are; else, and where
-    the call is traced (no addresses to pass), one GEMM each. A GEMM with W as its addend first copies W into its output and takes bf16 copies of both adapters:
-    168 us for the 4B layer's five projections against 51 (two launches)."""
+    the call's operators are recorded (``_recorded``), one GEMM each. A GEMM with W as its addend
+    first copies W into its output and takes bf16 copies of both adapters: 168 us for the 4B layer's
+    five projections against 51 (two launches)."""
     rank = a_s[0].shape[1]
     if (dtype == torch.bfloat16 and len(ws) <= _lib.MAX_MERGE and rank in (32, 64, 96, 128)
-            and not torch.compiler.is_compiling()
+            and not _recorded()
             and all(w.is_cuda and w.dtype == dtype and a.dtype == b.dtype == torch.float32 and w.shape[1] % 8 == 0
                     and w.numel() > 0 and a.device == b.device == w.device == ws[0].device
                     and a.shape == (w.shape[0], rank) and b.shape == (rank, w.shape[1])
