@@ -633,3 +633,36 @@ def test_no_stream_of_a_cpu_device():
 
     with pytest.raises(ValueError):
         _lib.current_stream(torch.device("cpu"))
+
+
+def test_kept_checks_and_plans_look_up_plain_values_only():
+    """What depends on the options' values is kept by those values: a numpy or tensor scalar is taken as its
+    value at the call (also after it was changed in place), a list raises what any wrong option raises."""
+    import numpy as np
+
+    from tjev_amd import _lib
+    from tjev_amd.gdn import _check, _plan
+    from tjev_amd.serve import _decode_dims, _decode_params
+
+    opts = ("high", "doubling", 16, 2 * 2 * 16 + 4 * 16, 2, 16, 4, 16, 0, None)
+    assert _check(*opts) == 1
+    assert _check(*opts[:4], np.array(2), *opts[5:]) == 1
+    with pytest.raises(ValueError, match="precision"):
+        _check(["high"], *opts[1:])
+    chunk = torch.tensor(16)
+    assert _check(*opts[:2], chunk, *opts[3:]) == 1
+    chunk.fill_(24)
+    with pytest.raises(ValueError, match="power-of-two"):
+        _check(*opts[:2], chunk, *opts[3:])
+
+    def plan(c, heads=2):
+        return _plan(_lib.load(), 1, 96, heads, 16, 4, 16, 4, c, torch.float32, torch.float32, "high", "doubling", 0, "states")
+
+    assert plan(16) is plan(16) and plan(32) is not plan(16)
+    chunk.fill_(16)
+    assert plan(chunk).n_chunks == 6
+    chunk.fill_(32)
+    assert plan(chunk).n_chunks == 3
+    assert plan(16, np.array(2)).params.key_heads == 2
+    assert _decode_dims(np.array(16), 16) == (None, 16)
+    _decode_params(1, np.array(2), 16, 4, 16, 4, torch.float32, torch.float32)

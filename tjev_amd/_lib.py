@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import functools
 from pathlib import Path
 
 import torch  # noqa: F401  (loads the HIP runtime the library binds to)
@@ -188,6 +189,22 @@ def open_library(path: Path) -> ctypes.CDLL:
     lib.tjev_gdn_lds_poison.restype = i32
     _OPENED[key] = lib
     return lib
+
+
+_PLAIN = frozenset((int, bool, float, str, type(None), torch.dtype, ctypes.CDLL))
+
+
+def by_value(fn):
+    """``fn`` with its results kept by its arguments' values (the latest 256), for functions that depend
+    on those alone. Arguments other than plain values, dtypes and libraries (a numpy or tensor scalar, a list)
+    may not be hashable or may change in place: such a call is not looked up, it runs ``fn``."""
+    kept = functools.lru_cache(maxsize=256, typed=True)(fn)
+
+    @functools.wraps(fn)
+    def call(*args):
+        return kept(*args) if _PLAIN.issuperset(map(type, args)) else fn(*args)
+
+    return call
 
 
 def current_stream(device: torch.device) -> int:

@@ -19,7 +19,6 @@ CPU tensor, the operator raises.
 from __future__ import annotations
 
 import ctypes
-import functools
 import math
 
 import torch
@@ -237,7 +236,7 @@ class GdnPlan:
         _lib.check_status(status)
 
 
-@functools.lru_cache(maxsize=256, typed=True)
+@_lib.by_value
 def _plan(lib, batch, length, key_heads, key_dim, value_heads, value_dim, taps, chunk, io_dtype, gate_dtype, precision,
           inverse, heads_per_step, residuals, qk_dtype=None) -> GdnPlan:
     """The plan of one problem shape on the library in use (``lib``, part of the key): a program
@@ -402,12 +401,15 @@ class _CoreCont(torch.autograd.Function):
 def _check(precision, inverse, chunk, width, key_heads, key_dim, value_heads, value_dim, heads_per_step,
            conv_weight):
     """gdn_megakernel's checks, in its order and wording (pallas_tpu_mega.py:597-615)."""
-    return _check_values(precision, inverse, chunk, width, key_heads, key_dim, value_heads, value_dim, heads_per_step,
-                         None if conv_weight is None else conv_weight.shape[0])
+    _check_values(precision, inverse, chunk, width, key_heads, key_dim, value_heads, value_dim, heads_per_step)
+    taps = 1 if conv_weight is None else conv_weight.shape[0]
+    if not 1 <= taps <= 5:
+        raise ValueError(f"conv kernel of {taps} taps: the megakernel supports 1..5")
+    return taps
 
 
-@functools.lru_cache(maxsize=256, typed=True)
-def _check_values(precision, inverse, chunk, width, key_heads, key_dim, value_heads, value_dim, heads_per_step, taps):
+@_lib.by_value
+def _check_values(precision, inverse, chunk, width, key_heads, key_dim, value_heads, value_dim, heads_per_step):
     if precision not in PRECISIONS:
         raise ValueError(f"precision in {PRECISIONS}")
     if inverse not in INVERSE_BLOCKS:
@@ -422,10 +424,6 @@ def _check_values(precision, inverse, chunk, width, key_heads, key_dim, value_he
     hb = heads_per_block(value_heads, ratio, heads_per_step or 8)
     if 3 * hb > LANES:
         raise ValueError(f"at most 42 heads per step, not {hb}")
-    taps = 1 if taps is None else taps
-    if not 1 <= taps <= 5:
-        raise ValueError(f"conv kernel of {taps} taps: the megakernel supports 1..5")
-    return taps
 
 
 def gdn_megakernel(qkv: torch.Tensor, a: torch.Tensor, b: torch.Tensor, a_log: torch.Tensor,

@@ -14,7 +14,6 @@ belongs to; a new request starts from a fresh prefill.
 from __future__ import annotations
 
 import ctypes
-import functools
 import math
 
 import torch
@@ -96,14 +95,14 @@ def gdn_prefill(qkv, a, b, a_log, dt_bias, conv_weight, segment_ids, *, key_head
     return out, state, conv_state
 
 
-@functools.lru_cache(maxsize=256, typed=True)
+@_lib.by_value
 def _decode_params(batch, key_heads, key_dim, value_heads, value_dim, taps, io_dtype, gate_dtype):
     """The library's view of a decode step's shape (a reference to the struct; never changed)."""
     return ctypes.byref(_lib.Params(batch, 1, key_heads, key_dim, value_heads, value_dim, taps, 64, _DTYPES[io_dtype],
                                     _DTYPES[gate_dtype], 1, 0, 0, 0))
 
 
-@functools.lru_cache(maxsize=256, typed=True)
+@_lib.by_value
 def _decode_dims(key_dim, value_dim):
     return value_groups(key_dim, value_dim), run_dim(key_dim, value_dim)
 
