@@ -666,3 +666,18 @@ def test_kept_checks_and_plans_look_up_plain_values_only():
     assert plan(16, np.array(2)).params.key_heads == 2
     assert _decode_dims(np.array(16), 16) == (None, 16)
     _decode_params(1, np.array(2), 16, 4, 16, 4, torch.float32, torch.float32)
+
+
+def test_a_kept_plan_runs_on_the_library_it_is_kept_under():
+    """The library in use can change between the lookup and the plan's construction (another thread enters
+    or leaves ``_lib.library``): the plan still holds the library it was asked for."""
+    from tjev_amd import _lib
+    from tjev_amd.gdn import _plan
+
+    poison = _lib.open_library(_lib.LDS_POISON_PATH)
+    args = (1, 48, 2, 16, 4, 16, 4, 16, torch.float32, torch.float32, "high", "doubling", 0, "states")
+    assert _plan(poison, *args).lib is poison
+    assert _plan(_lib.load(), *args).lib is _lib.load()
+    # an error's message comes from the library that refused the call (a shape it does not hold)
+    with pytest.raises((_lib.GdnLibraryError, ValueError), match="no kernels for chunk 16, head dim 32"):
+        _plan(poison, 1, 48, 2, 32, 4, 32, *args[6:])

@@ -216,9 +216,10 @@ def current_stream(device: torch.device) -> int:
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
-def check_status(status: int) -> None:
+def check_status(status: int, lib: ctypes.CDLL | None = None) -> None:
+    """Raises for a nonzero status of a call into ``lib`` (the library in use when not given)."""
     if status != 0:
-        raise GdnLibraryError(status, load().tjev_gdn_last_error().decode())
+        raise GdnLibraryError(status, (load() if lib is None else lib).tjev_gdn_last_error().decode())
 
 
 class KernelTimer:

@@ -137,8 +137,8 @@ class GdnPlan:
     def __init__(self, *, batch: int, length: int, key_heads: int, key_dim: int, value_heads: int,
                  value_dim: int, taps: int, chunk: int, io_dtype: torch.dtype,
                  gate_dtype: torch.dtype, precision: str = "high", inverse: str = "doubling",
-                 heads_per_step: int = 0, residuals: str = "states"):
-        self.lib = _lib.load()
+                 heads_per_step: int = 0, residuals: str = "states", lib: ctypes.CDLL | None = None):
+        self.lib = _lib.load() if lib is None else lib
         if io_dtype not in _DTYPES or gate_dtype not in _DTYPES:
             raise ValueError(f"the GDN megakernel takes float32 or bfloat16 tensors, not {io_dtype}/{gate_dtype}")
         if residuals not in _lib.RESIDUALS:
@@ -149,7 +149,7 @@ class GdnPlan:
         status = self.lib.tjev_gdn_check(ctypes.byref(self.params))
         if status == 1:
             raise ValueError(self.lib.tjev_gdn_last_error().decode())
-        _lib.check_status(status)
+        _lib.check_status(status, self.lib)
         self.chunk_run = min(max(chunk, 16), 128)  # the kernels' chunk (tjev_gdn_params.chunk clamped)
         self.n_chunks = math.ceil(length / self.chunk_run)
         self.states_shape = (batch, value_heads, self.n_chunks, key_dim, value_dim)
@@ -195,7 +195,7 @@ class GdnPlan:
             ctypes.byref(self.params), self._stream(qkv.device), _ptr(qkv), _ptr(a), _ptr(b), _ptr(a_log),
             _ptr(dt_bias), _ptr(conv_w), _ptr(seg), _ptr(out), _ptr(residuals), _ptr(workspace),
             workspace.numel())
-        _lib.check_status(status)
+        _lib.check_status(status, self.lib)
 
     def forward_normed(self, qkv, a, b, a_log, dt_bias, conv_w, seg, gate, norm_weight, eps: float, out, y,
                        residuals, workspace) -> None:
@@ -206,7 +206,7 @@ class GdnPlan:
             _ptr(dt_bias), _ptr(conv_w), _ptr(seg), None, None, _ptr(gate), _ptr(norm_weight),
             ctypes.c_float(eps), _ptr(out), _ptr(y), _ptr(residuals), None, None, _ptr(workspace),
             workspace.numel())
-        _lib.check_status(status)
+        _lib.check_status(status, self.lib)
 
     def normed_bwd_bytes(self, norm_weight_grad: bool) -> int:
         want = bool(norm_weight_grad)
@@ -225,7 +225,7 @@ class GdnPlan:
             _ptr(norm_weight), ctypes.c_float(eps), _ptr(d_y), None, _ptr(d_qkv), _ptr(d_a), _ptr(d_b),
             _ptr(d_a_log), _ptr(d_dt_bias), _ptr(d_conv_w), None, None, _ptr(d_gate), _ptr(d_norm_weight),
             _ptr(workspace), workspace.numel())
-        _lib.check_status(status)
+        _lib.check_status(status, self.lib)
 
     def backward(self, qkv, a, b, a_log, dt_bias, conv_w, seg, residuals, d_out, d_qkv, d_a, d_b, d_a_log,
                  d_dt_bias, d_conv_w, workspace) -> None:
@@ -233,7 +233,7 @@ class GdnPlan:
             ctypes.byref(self.params), self._stream(qkv.device), _ptr(qkv), _ptr(a), _ptr(b), _ptr(a_log),
             _ptr(dt_bias), _ptr(conv_w), _ptr(seg), _ptr(residuals), _ptr(d_out), _ptr(d_qkv), _ptr(d_a),
             _ptr(d_b), _ptr(d_a_log), _ptr(d_dt_bias), _ptr(d_conv_w), _ptr(workspace), workspace.numel())
-        _lib.check_status(status)
+        _lib.check_status(status, self.lib)
 
 
 @_lib.by_value
@@ -245,7 +245,7 @@ def _plan(lib, batch, length, key_heads, key_dim, value_heads, value_dim, taps, 
     threads share them."""
     plan = GdnPlan(batch=batch, length=length, key_heads=key_heads, key_dim=key_dim, value_heads=value_heads,
                    value_dim=value_dim, taps=taps, chunk=chunk, io_dtype=io_dtype, gate_dtype=gate_dtype,
-                   precision=precision, inverse=inverse, heads_per_step=heads_per_step, residuals=residuals)
+                   precision=precision, inverse=inverse, heads_per_step=heads_per_step, residuals=residuals, lib=lib)
     if qk_dtype is not None:
         plan.params.qk_dtype = _DTYPES[qk_dtype]
     return plan
