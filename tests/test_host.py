@@ -681,3 +681,22 @@ def test_a_kept_plan_runs_on_the_library_it_is_kept_under():
     # an error's message comes from the library that refused the call (a shape it does not hold)
     with pytest.raises((_lib.GdnLibraryError, ValueError), match="no kernels for chunk 16, head dim 32"):
         _plan(poison, 1, 48, 2, 32, 4, 32, *args[6:])
+
+
+def _device_ir(c, d, part):
+    """The optimized LLVM IR of one gdn_inst.hip object's kernels."""
+    from tjev_amd.build import CSRC, FLAGS, _hipcc, unit_flags
+
+    cmd = [_hipcc(), *FLAGS, *unit_flags(c, d, part), "--cuda-device-only", "-emit-llvm", "-S", "-o", "-", "-c",
+           str(CSRC / "gdn_inst.hip")]
+    return subprocess.run(cmd, capture_output=True, text=True, check=True).stdout
+
+
+@pytest.mark.parametrize("chunk", [16, 32, 64, 128])
+def test_output_kernel_keeps_no_private_arrays(chunk):
+    """At head dim 16 the output kernel's operands all stay in registers, in every precision (an array left in
+    private memory is moved to LDS and more than doubled the kernel's time)."""
+    ir = _device_ir(chunk, 16, 3)
+    kernels = re.findall(r"^define .*amdgpu_kernel void @(\w*k_out\w*)", ir, flags=re.M)
+    assert len(kernels) == 16
+    assert [line.strip() for line in ir.splitlines() if " = alloca " in line] == []
