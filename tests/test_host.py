@@ -700,3 +700,16 @@ def test_output_kernel_keeps_no_private_arrays(chunk):
     kernels = re.findall(r"^define .*amdgpu_kernel void @(\w*k_out\w*)", ir, flags=re.M)
     assert len(kernels) == 16
     assert [line.strip() for line in ir.splitlines() if " = alloca " in line] == []
+
+
+def test_chunk_16_at_head_dim_128_holds_half_a_state():
+    """The output kernel of one wave per workgroup stages its 128 x 128 state in halves of 128 registers per thread:
+    no instance spills as many (a whole state held as the prefetch spilled up to 360)."""
+    from tjev_amd.build import CSRC, FLAGS, _hipcc, unit_flags
+
+    cmd = [_hipcc(), *FLAGS, *unit_flags(16, 128, 3), "--cuda-device-only", "-Rpass-analysis=kernel-resource-usage", "-o", "/dev/null",
+           "-c", str(CSRC / "gdn_inst.hip")]
+    remarks = subprocess.run(cmd, capture_output=True, text=True, check=True).stderr
+    names = re.findall(r"Function Name: (\S*k_out\S*)", remarks)
+    spills = [int(n) for n in re.findall(r" VGPRs Spill: (\d+)", remarks)]
+    assert len(names) == len(spills) == 16 and max(spills) < 128, dict(zip(names, spills))

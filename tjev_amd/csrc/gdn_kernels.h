@@ -1188,6 +1188,17 @@ struct RawV {
 template <int C, int D, int PI>
 constexpr int wgs_per_cu() { return C == 64 && D == 128 && PI != P_F32 ? 2 : 1; }
 
+// In how many parts of its rows (or columns) the chunk kernels stage a D x D state: in halves for two
+// workgroups per CU, and where one wave loads it alone (a chunk of 16 at D = 128). There a whole state is
+// 256 registers per thread, held across a unit as its prefetch: k_out and k_chunk's backward modes spilled
+// up to 360 VGPRs, and each change of the instructions around them moved their times by up to a
+// third. In halves they spill 92 at most. Two rows of 1777 tokens, 32 heads, high, bf16 I/O: k_out 1060 (at
+// its worst since 1170) -> 489 us, with the norm 1390 (1650) -> 616, k_chunk backward 887 (1205) -> 553;
+// mixed 513 (560) -> 326, 566 (718) -> 390 and 372 (427) -> 341. A chunk of 32 (two waves, 128 registers)
+// keeps whole states: it spills nothing there.
+template <int C, int D>
+constexpr int state_parts(int wgs) { return wgs == 2 || (C == 16 && D == 128) ? 2 : 1; }
+
 // ---------------------------------------------------------------- k_chunk
 // Persistent over the (row, head, chunk) units as k_out; C/16 waves (one 16-row strip each).
 // MODE 0 (forward): writes w and u; MODE 2: also T (kept as a residual). MODE 1 (backward
@@ -1207,7 +1218,7 @@ __global__ __launch_bounds__(C * 4, (wgs_per_cu<C, D, PI>())) void k_chunk(GdnAr
   constexpr bool STORE_T = MODE == 1 || MODE == 2;
   constexpr int NT = C * 4;
   constexpr int LT = C + 4;
-  constexpr int NH = wgs_per_cu<C, D, PI>();  // S is staged in NH parts of its dk rows
+  constexpr int NH = state_parts<C, D>(wgs_per_cu<C, D, PI>());  // S is staged in NH parts of its dk rows
   using TR = OpTile<PI, C, D>;                // k rows
   using TK = OpTile<PI, D, C>;                // kbe^T, (v beta)^T, Y^T
   using TS = OpTile<PI, D, D / NH>;           // S^T, of one part
@@ -2197,7 +2208,7 @@ template <int C, int D, int PI, int PS, class TIO, bool NORM = false, bool FQ = 
 __global__ __launch_bounds__(C * 4, (wgs_per_cu<C, D, PI>())) void k_out(GdnArgs A) {
   constexpr int NT = C * 4;
   constexpr int LI = C + 4;
-  constexpr int NH = wgs_per_cu<C, D, PI>();  // S is staged in NH parts of its dk rows
+  constexpr int NH = state_parts<C, D>(wgs_per_cu<C, D, PI>());  // S is staged in NH parts of its dk rows
   using TR = OpTile<PI, C, D>;                // k rows
   using TK = OpTile<PI, D, C>;                // v_new^T
   using TS = OpTile<PI, D, D / NH>;           // S^T, of one part
@@ -2778,7 +2789,7 @@ template <int C, int D, int PI, int PS, class TIO>
 __global__ __launch_bounds__(C * 4, (wgs_per_cu<C, D, PI>())) void k_bwd_grads(GdnArgs A) {
   constexpr int NT = C * 4;
   constexpr int LA = C + 4;
-  constexpr int NH = wgs_per_cu<C, D, PI>();  // S and G are staged in NH parts of their columns
+  constexpr int NH = state_parts<C, D>(wgs_per_cu<C, D, PI>());  // S and G are staged in NH parts of their columns
   constexpr int TD = D / 16;
   constexpr int TC = C / 16;
   using TR = OpTile<PI, C, D>;       // v_new rows
