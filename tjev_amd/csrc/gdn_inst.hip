@@ -14,9 +14,12 @@
 #if GDN_PART == 2 || GDN_PART == 3 || GDN_PART == 4
 #define GDN_LANE_OFF32 1
 #endif
-// fragments converted value by value in k_bwd_grads: by pairs it spills 27 VGPRs instead of 11
-// (bf16 I/O at C = D = 128: 360 against 333 us)
-#if GDN_PART == 5
+// k_bwd_grads at D = 128 and chunks of 64 and 128 converts its fragments value by value: by pairs it
+// runs out of registers at "high" (bf16 I/O, two rows of 1777 tokens, 32 heads: 165 us against 174 at C =
+// 128, 155 against 159 at C = 64; 333 against 360 at the 0.8B layer shape; the other modes and fp32 I/O
+// within 4% either way). Everywhere else pairs take the same time within 2%, or less (C = D = 32, high:
+// 30.8 us against 34.4; C = 32, D = 16: 24.1 against 27.0).
+#if GDN_PART == 5 && GDN_D == 128 && GDN_C >= 64
 #define GDN_FRAG_PAIRS 0
 #endif
 #include "gdn_kernels.h"
