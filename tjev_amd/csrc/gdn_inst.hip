@@ -85,7 +85,7 @@ GDN_EACH_PAIR(GDN_CHUNK_FV)
 #if GDN_C >= 64 && GDN_D == 128  // the bf16 modes on four compute waves
 #define GDN_SCAN_FWD(PI, PS)
 #if GDN_C == 128
-GDN_KW_2 __global__ void k_scan_fwd_split<P_F32, P_F32>(GdnArgs);
+GDN_KW_2 __global__ void k_scan_fwd_split<128>(GdnArgs);
 #else
 GDN_KW_2 __global__ void k_scan_fwd<GDN_C, GDN_D, kDVT, P_F32, P_F32>(GdnArgs);
 #endif
@@ -124,10 +124,10 @@ GDN_EACH_PAIR(GDN_GRADS)
 #if GDN_PART == 0
 namespace {
 
-// compute units of the current device (queried once per device): the persistent kernels run
-// one workgroup per CU
 dim3 chunks_grid(const GdnArgs& A) { return dim3(A.B * A.H * A.N); }
 
+// compute units of the current device (queried once per device): the persistent kernels run
+// wgs_per_cu() workgroups on each
 int cu_count() {
   static int cache[16] = {0};
   int dev = 0;
@@ -164,10 +164,8 @@ hipError_t run(const GdnArgs& A, hipStream_t st, int backward, const Timer* tm) 
   // kernels to build them: fail rather than let k_prep write through a null pointer
   if (!backward && ((!L.fuse_v && !A.vv) || (!L.fuse_q && !A.qn))) return hipErrorInvalidValue;
   const dim3 tiles(chains * parts);
-  const int units = A.B * A.H * A.N, cus = cu_count();
-  const dim3 persist(units < cus ? units : cus);
-  const int room = wgs_per_cu<C, D, PI>() * cus;
-  const dim3 persist_two(units < room ? units : room);
+  const int units = A.B * A.H * A.N, room = wgs_per_cu<C, D, PI>() * cu_count();
+  const dim3 persist(units < room ? units : room);
   auto mark = [&](int k, int end) {
     if (tm) tm->mark(tm->self, k, end, st);
   };
@@ -183,42 +181,42 @@ hipError_t run(const GdnArgs& A, hipStream_t st, int backward, const Timer* tm) 
     if (A.res == 0) {
       if (L.fuse_v) {
         if constexpr (kFV) {
-          if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, true, true>), persist_two, dim3(C * 4));
-          else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, false, true>), persist_two, dim3(C * 4));
+          if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, true, true>), persist, dim3(C * 4));
+          else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, false, true>), persist, dim3(C * 4));
         }
-      } else if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, true>), persist_two, dim3(C * 4));
-      else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, false>), persist_two, dim3(C * 4));
+      } else if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, true>), persist, dim3(C * 4));
+      else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, false>), persist, dim3(C * 4));
     } else {  // T kept for the backward
       if (L.fuse_v) {
         if constexpr (kFV) {
-          if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, true, true>), persist_two, dim3(C * 4));
-          else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, false, true>), persist_two, dim3(C * 4));
+          if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, true, true>), persist, dim3(C * 4));
+          else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, false, true>), persist, dim3(C * 4));
         }
-      } else if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, true>), persist_two, dim3(C * 4));
-      else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, false>), persist_two, dim3(C * 4));
+      } else if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, true>), persist, dim3(C * 4));
+      else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, false>), persist, dim3(C * 4));
     }
     if constexpr (C >= 64 && D == 128 && PI != P_F32) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_quad<C, PI, PS>), tiles, dim3(512));
-    else if constexpr (C == 128 && D == 128) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_split<PI, PS>), tiles, dim3(512));
+    else if constexpr (C == 128 && D == 128) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_split<C>), tiles, dim3(512));
     else GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd<C, D, DVT, PI, PS>), tiles, dim3(NS));
     if (L.fuse_q) {
       if constexpr (kFV) {
-        if (A.ny) GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO, true, true>), persist_two, dim3(C * 4));
-        else GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO, false, true>), persist_two, dim3(C * 4));
+        if (A.ny) GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO, true, true>), persist, dim3(C * 4));
+        else GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO, false, true>), persist, dim3(C * 4));
       }
-    } else if (A.ny) GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO, true>), persist_two, dim3(C * 4));
-    else GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO>), persist_two, dim3(C * 4));
+    } else if (A.ny) GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO, true>), persist, dim3(C * 4));
+    else GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO>), persist, dim3(C * 4));
     if (const unsigned tail = tail_blocks<D, TIO>(A)) GDN_LAUNCH(K_FINAL_STATE, (k_tail<C, D, TIO>), dim3(tail), dim3(256));
   } else {
     const int wouts = A.d_conv_w ? A.taps * A.W : 0;  // one workgroup per head, then the conv weights
     if (A.taps <= 4) GDN_LAUNCH(K_PREP_BWD, (k_prep<C, D, TIO, TG, 3>), prep, dim3(256));
     else GDN_LAUNCH(K_PREP_BWD, (k_prep<C, D, TIO, TG, 4>), prep, dim3(256));
     if (A.res == 0) {  // T and v_new rebuilt
-      if (A.inv == 0) GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 1, true>), persist_two, dim3(C * 4));
-      else GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 1, false>), persist_two, dim3(C * 4));
+      if (A.inv == 0) GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 1, true>), persist, dim3(C * 4));
+      else GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 1, false>), persist, dim3(C * 4));
     } else if (A.res == 1) {  // v_new from the saved T
-      GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 3, false>), persist_two, dim3(C * 4));
+      GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 3, false>), persist, dim3(C * 4));
     }  // else both saved
-    GDN_LAUNCH(K_BWD_LOCAL, (k_bwd_local<C, D, PI, TIO>), persist_two, dim3(C * 4));
+    GDN_LAUNCH(K_BWD_LOCAL, (k_bwd_local<C, D, PI, TIO>), persist, dim3(C * 4));
     GDN_LAUNCH(K_SCAN_BWD, (k_scan_bwd<C, D, DVT, PI, PS, TIO>), tiles, dim3(NS));
     GDN_LAUNCH(K_BWD_GRADS, (k_bwd_grads<C, D, PI, PS, TIO>), chunks, dim3(C * 4));
     // the conv halo sized to the taps (taps - 1 <= 3 for the model's conv of 4); d(conv w)
@@ -251,10 +249,8 @@ hipError_t run_v2(const GdnArgs& A, hipStream_t st, int backward, const Timer* t
   L.fuse_v = 0;  // v is an input here (k_prep_v2 writes its rows)
   L.fuse_q = 0;
   const dim3 tiles(chains * parts);
-  const int units = A.B * A.H * A.N, cus = cu_count();
-  const dim3 persist(units < cus ? units : cus);
-  const int room = wgs_per_cu<C, D, PI>() * cus;
-  const dim3 persist_two(units < room ? units : room);
+  const int units = A.B * A.H * A.N, room = wgs_per_cu<C, D, PI>() * cu_count();
+  const dim3 persist(units < room ? units : room);
   auto mark = [&](int k, int end) {
     if (tm) tm->mark(tm->self, k, end, st);
   };
@@ -267,26 +263,26 @@ hipError_t run_v2(const GdnArgs& A, hipStream_t st, int backward, const Timer* t
   if (!backward) {
     GDN_LAUNCH(K_PREP_FWD, (k_prep_v2<C, D, TIO, TQK, TG>), ends, dim3(256));
     if (A.res == 0) {
-      if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, true>), persist_two, dim3(C * 4));
-      else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, false>), persist_two, dim3(C * 4));
+      if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, true>), persist, dim3(C * 4));
+      else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 0, false>), persist, dim3(C * 4));
     } else {
-      if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, true>), persist_two, dim3(C * 4));
-      else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, false>), persist_two, dim3(C * 4));
+      if (A.inv == 0) GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, true>), persist, dim3(C * 4));
+      else GDN_LAUNCH(K_CHUNK_FWD, (k_chunk<C, D, PI, PS, 2, false>), persist, dim3(C * 4));
     }
     if constexpr (C >= 64 && D == 128 && PI != P_F32) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_quad<C, PI, PS>), tiles, dim3(512));
-    else if constexpr (C == 128 && D == 128) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_split<PI, PS>), tiles, dim3(512));
+    else if constexpr (C == 128 && D == 128) GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd_split<C>), tiles, dim3(512));
     else GDN_LAUNCH(K_SCAN_FWD, (k_scan_fwd<C, D, DVT, PI, PS>), tiles, dim3(NS));
-    GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO>), persist_two, dim3(C * 4));
+    GDN_LAUNCH(K_OUT, (k_out<C, D, PI, PS, TIO>), persist, dim3(C * 4));
     if (const unsigned tail = tail_blocks<D, TIO>(A)) GDN_LAUNCH(K_FINAL_STATE, (k_tail<C, D, TIO>), dim3(tail), dim3(256));
   } else {
     GDN_LAUNCH(K_PREP_BWD, (k_prep_v2<C, D, TIO, TQK, TG>), ends, dim3(256));
     if (A.res == 0) {
-      if (A.inv == 0) GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 1, true>), persist_two, dim3(C * 4));
-      else GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 1, false>), persist_two, dim3(C * 4));
+      if (A.inv == 0) GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 1, true>), persist, dim3(C * 4));
+      else GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 1, false>), persist, dim3(C * 4));
     } else if (A.res == 1) {
-      GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 3, false>), persist_two, dim3(C * 4));
+      GDN_LAUNCH(K_CHUNK_BWD, (k_chunk<C, D, PI, PS, 3, false>), persist, dim3(C * 4));
     }
-    GDN_LAUNCH(K_BWD_LOCAL, (k_bwd_local<C, D, PI, TIO>), persist_two, dim3(C * 4));
+    GDN_LAUNCH(K_BWD_LOCAL, (k_bwd_local<C, D, PI, TIO>), persist, dim3(C * 4));
     GDN_LAUNCH(K_SCAN_BWD, (k_scan_bwd<C, D, DVT, PI, PS, TIO>), tiles, dim3(NS));
     GDN_LAUNCH(K_BWD_GRADS, (k_bwd_grads<C, D, PI, PS, TIO>), chunks_grid(A), dim3(C * 4));
     GDN_LAUNCH(K_POST, (k_post_v2<C, D, TIO, TQK, TG>), ends, dim3(256));

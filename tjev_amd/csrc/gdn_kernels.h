@@ -1558,8 +1558,8 @@ __global__ __launch_bounds__((C > D ? C : D) * 4) void k_scan_fwd(GdnArgs A) {
 }
 
 // ---------------------------------------------------------------- k_scan_fwd_split
-// The forward scan at C = D = 128 in the fp32 mode (the bf16 modes: k_scan_fwd_quad), with its two products chained in registers. Two compute
-// waves each own 16 value columns of the 32-column Dv tile: S[:, cols] (Dk x 16, 8 accumulator
+// The forward scan at C = D = 128 in the fp32 mode (the bf16 modes: k_scan_fwd_quad), with its two
+// products chained in registers. Two compute waves each own 16 value columns of the 32-column Dv tile: S[:, cols] (Dk x 16, 8 accumulator
 // tiles, rows dk) and v_new[:, cols] (C x 16, 8 tiles, rows tokens). Per chunk:
 //   P1  v_new = u + (-w) S             A: -w (LDS, rows tokens), B: S from the accumulators
 //   P2  S = carry S + k^T (kws v_new)  A: k^T (LDS, rows dk), B: v_new from the accumulators,
@@ -1574,10 +1574,6 @@ __global__ __launch_bounds__((C > D ? C : D) * 4) void k_scan_fwd(GdnArgs A) {
 // its columns of the u^T buffer once it has read u from there, and in P2 each loader thread
 // stores the values it then overwrites with the next u^T. Two barriers per chunk. Same chunk
 // ranges, replays and outputs as k_scan_fwd.
-struct ScanSplitBuf {
-  static constexpr int C = 128, D = 128, DVT = 32, LU = C + 4;
-};
-
 // B fragment values (rows 8 (lane/16) .. + 7 of the 32-row contraction step, column lane % 16)
 // from accumulator tiles t0 (rows 0-15) and t1 (rows 16-31)
 __device__ __forceinline__ void acc_pair_to_b(const f32x4& t0, const f32x4& t1, float (&v)[8]) {
@@ -1599,19 +1595,18 @@ __device__ __forceinline__ void acc_pair_to_b(const f32x4& t0, const f32x4& t1, 
 // operand tile (8 row tiles), B from the accumulator tiles bsrc (two per 32-deep step). Each
 // step's eight A fragments are read one step ahead, so the LDS latency runs under the previous
 // step's MFMAs.
-template <int P, class OP>
-__device__ __forceinline__ void split_product(f32x4 (&acc)[8], const OP& a, const f32x4 (&bsrc)[8],
+__device__ __forceinline__ void split_product(f32x4 (&acc)[8], const Op<P_F32>& a, const f32x4 (&bsrc)[8],
                                               const float* bscale = nullptr) {
   const int r = lane() & 15, kg = (lane() >> 4) << 3;
-  Frag<a_prec<P>()> fa[2][8];
+  Frag<P_F32> fa[2][8];
 #pragma unroll
-  for (int t = 0; t < 8; ++t) fa[0][t] = a.template frag<a_prec<P>()>(16 * t + r, kg);
+  for (int t = 0; t < 8; ++t) fa[0][t] = a.frag<P_F32>(16 * t + r, kg);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
     if (s + 1 < 4) {
 #pragma unroll
-      for (int t = 0; t < 8; ++t) fa[(s + 1) & 1][t] = a.template frag<a_prec<P>()>(16 * t + r, 32 * (s + 1) + kg);
+      for (int t = 0; t < 8; ++t) fa[(s + 1) & 1][t] = a.frag<P_F32>(16 * t + r, 32 * (s + 1) + kg);
     }
     // the scheduler would otherwise sink these reads next to their MFMAs (register pressure)
     __builtin_amdgcn_sched_barrier(0);
@@ -1623,18 +1618,19 @@ __device__ __forceinline__ void split_product(f32x4 (&acc)[8], const OP& a, cons
       bv[0] *= s0.x; bv[1] *= s0.y; bv[2] *= s0.z; bv[3] *= s0.w;
       bv[4] *= s1.x; bv[5] *= s1.y; bv[6] *= s1.z; bv[7] *= s1.w;
     }
-    const Frag<b_prec<P>()> fb = make_frag<b_prec<P>()>(bv);
+    const Frag<P_F32> fb = make_frag<P_F32>(bv);
 #pragma unroll
-    for (int t = 0; t < 8; ++t) mma<P>(acc[t], fa[s & 1][t], fb);
+    for (int t = 0; t < 8; ++t) mma<P_F32>(acc[t], fa[s & 1][t], fb);
   }
 }
 
-template <int PI, int PS>
+template <int C>
 __global__ __launch_bounds__(512) void k_scan_fwd_split(GdnArgs A) {
-  constexpr int C = 128, D = 128, DVT = 32, NT = 512, LU = C + 4;
+  static_assert(C == 128, "the staging slots below");
+  constexpr int D = 128, DVT = 32, NT = 512, LU = C + 4;
   constexpr int NL = NT - 128;      // loader threads (waves 2 .. 7)
-  using TW = OpTile<PI, C, D>;      // -w: A(i = token, k = dk)
-  using TK = OpTile<PI, D, C>;      // k^T: A(i = dk, k = token)
+  using TW = OpTile<P_F32, C, D>;   // -w: A(i = token, k = dk)
+  using TK = OpTile<P_F32, D, C>;   // k^T: A(i = dk, k = token)
   __shared__ __align__(16) char sW[TW::BYTES];
   __shared__ __align__(16) char sK[TK::BYTES];
   __shared__ __align__(16) float sU[DVT * LU];  // u^T: [value column][token]
@@ -1642,7 +1638,7 @@ __global__ __launch_bounds__(512) void k_scan_fwd_split(GdnArgs A) {
   __shared__ float scarry[2];
   __shared__ int red[NT / 64];
   GDN_POISON_LDS(sW, sK, sU, skws, scarry, red);
-  const Op<PI> ow = TW::at(sW), okt = TK::at(sK);
+  const Op<P_F32> ow = TW::at(sW), okt = TK::at(sK);
   const ScanIx ix(A);
   const int tile = ix.tile, bh = ix.bh, part = ix.part;
   const int h = bh % A.H, b = bh / A.H, hk = h / A.ratio;
@@ -1712,22 +1708,15 @@ __global__ __launch_bounds__(512) void k_scan_fwd_split(GdnArgs A) {
     }
   };
   auto store_s = [&](int n) {  // S before chunk n, from sU, where put_u writes next
-    StateT<PS>* sg = states_ptr<PS>(A) + ((size_t)bh * A.N + n) * D * D + j0;
+    float* sg = states_ptr<P_F32>(A) + ((size_t)bh * A.N + n) * D * D + j0;
 #pragma unroll
     for (int it = 0; it < 3; ++it) {
       const int idx = lt + it * NL;
       if (idx < 1024) {
         const int dk = idx >> 3, c = 4 * (idx & 7);
-        if constexpr (sizeof(StateT<PS>) == 2) {  // and the final state's fp32 source
-          const float v[4] = {sU[(c + 0) * LU + dk], sU[(c + 1) * LU + dk], sU[(c + 2) * LU + dk],
-                              sU[(c + 3) * LU + dk]};
-          st4_io(sg + (unsigned)(dk * D + c), v);
-          if (n == A.N - 1 && A.s_last) st4_io(A.s_last + (size_t)bh * D * D + j0 + (unsigned)(dk * D + c), v);
-        } else {
-          const float4 v = make_float4(sU[(c + 0) * LU + dk], sU[(c + 1) * LU + dk], sU[(c + 2) * LU + dk],
-                                       sU[(c + 3) * LU + dk]);
-          *reinterpret_cast<float4*>(sg + (unsigned)(dk * D + c)) = v;
-        }
+        const float4 v = make_float4(sU[(c + 0) * LU + dk], sU[(c + 1) * LU + dk], sU[(c + 2) * LU + dk],
+                                     sU[(c + 3) * LU + dk]);
+        *reinterpret_cast<float4*>(sg + (unsigned)(dk * D + c)) = v;
       }
     }
   };
@@ -1787,12 +1776,12 @@ __global__ __launch_bounds__(512) void k_scan_fwd_split(GdnArgs A) {
       for (int dt = 0; dt < 8; ++dt)
         *reinterpret_cast<float4*>(sU + (16 * jt + acc_col()) * LU + 16 * dt + acc_row(0)) =
             make_float4(accS[dt][0], accS[dt][1], accS[dt][2], accS[dt][3]);
-      split_product<PS>(accV, ow, accS);
+      split_product(accV, ow, accS);
       __syncthreads();  // (k kws)^T of chunk n staged
       const float carry = scarry[n & 1];
 #pragma unroll
       for (int dt = 0; dt < 8; ++dt) accS[dt] *= carry;
-      split_product<PI>(accS, okt, accV, skws[n & 1]);  // S = carry S + k^T (kws v_new)
+      split_product(accS, okt, accV, skws[n & 1]);  // S = carry S + k^T (kws v_new)
       if (emit) {
         float* vg = A.vnew + hoff(A, b, h, A.H, n, C, D) + col;
 #pragma unroll
