@@ -1,6 +1,6 @@
 """The model head dimension (Dk = Dv = 128, chunk 128) at every precision (GPU): the chunk
-kernels and the forward scan at this shape (its own kernel, k_scan_fwd_split) under fp32
-("highest") against the fp64 oracle at the fp32 bar, with packed segments (the scans' chunk
+kernels and the forward scan at this shape (its own kernels: k_scan_fwd_split in fp32,
+k_scan_fwd_quad in the bf16 modes) under fp32 ("highest") against the fp64 oracle at the fp32 bar, with packed segments (the scans' chunk
 ranges split at resets) and trailing padding; "mixed" and one-pass "bf16" at the bars of the
 small-head precision test; a row run in two calls (initial state and conv history) equal to
 the row run at once.

@@ -15,7 +15,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from gdn_cases import NAMES, case_inputs, cosine, hip_outputs, rel
+from gdn_cases import NAMES, case_inputs, cosine, hip_outputs, rel, rel_l2
 
 pytestmark = pytest.mark.gpu
 
@@ -37,6 +37,29 @@ def test_residual_policies_agree(precision, dtype):
             assert cosine(runs["all"][k], runs["states"][k]) >= 0.999999, k
             if dtype == torch.float32 and k not in ("A_log", "dt_bias"):
                 assert rel(runs["all"][k], runs["states"][k]) <= 1e-5, k
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("precision", ["high", "mixed", "bf16"])
+@pytest.mark.parametrize("C", [16, 64])
+def test_residual_policies_agree_where_states_are_staged_in_halves(C, precision, dtype):
+    """Head dim 128 at chunks of 16 and 64 (a ragged last chunk, segment cuts off the chunk ends): the chunk
+    kernel that reads a kept T and the one that rebuilds it give the same results bit for bit, and v_new from the
+    forward's scan the same output; its gradients agree to the rounding of v_new's two ways (fp32 I/O: the
+    bars of the products, 1e-4 at three bf16 passes, 2e-2 at one)."""
+    shape = dict(key_heads=1, key_dim=128, value_heads=2, value_dim=128)
+    inputs, cot = case_inputs(2, 301, 1, 2, 128, cuts=[20, 64, 193], dtype=dtype, seed=11)
+    print(f"chunk {C} {precision} {dtype}", flush=True)
+    runs = {mode: hip_outputs(inputs, cot, chunk=C, precision=precision, residuals=mode, **shape)
+            for mode in ("states", "tinv", "all")}
+    print("all vs states", {k: f"{rel_l2(runs['all'][k], runs['states'][k]):.1e}" for k in runs["all"]}, flush=True)
+    for k in runs["states"]:
+        assert bool(torch.isfinite(runs["states"][k]).all()), k
+        assert torch.equal(runs["tinv"][k], runs["states"][k]), k
+    assert torch.equal(runs["all"]["out"], runs["states"]["out"])
+    for k in ("qkv", "a", "b", "w"):
+        tol = (1e-4 if precision == "high" else 2e-2) if dtype == torch.float32 else 2e-2
+        assert rel_l2(runs["all"][k], runs["states"][k]) <= tol, k
 
 
 def _kept_tinv(inputs, C, precision, inverse):
@@ -131,10 +154,10 @@ def test_states_are_bf16_when_the_state_products_are_one_pass(precision, dim):
     final state a run one chunk shorter returns. That final state is built from an fp32 copy of
     its last chunk's state (built from the bf16 residual instead, about half of its elements
     would round to another bf16 value). That holds bit for bit under "mixed", whose scan updates
-    the state with bf16x3 products (k_final_state: fp32); under "bf16" the scan's one-pass
+    the state with bf16x3 products (k_tail: fp32); under "bf16" the scan's one-pass
     update itself is that far from the final state's fp32 one (measured: 57% of the elements
-    equal), so there the two only agree to the mode's accuracy. dim 128 runs the two-wave
-    forward scan, dim 64 the generic one."""
+    equal), so there the two only agree to the mode's accuracy. dim 128 runs the four-wave
+    forward scan (k_scan_fwd_quad), dim 64 the generic one."""
     import ctypes
 
     from oracle.gdn_oracle import chunk_gated_delta_rule, core_inputs
