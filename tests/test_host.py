@@ -664,7 +664,7 @@ def test_kept_checks_and_plans_look_up_plain_values_only():
     chunk.fill_(32)
     assert plan(chunk).n_chunks == 3
     assert plan(16, np.array(2)).params.key_heads == 2
-    assert _decode_dims(np.array(16), 16) == (None, 16)
+    assert _decode_dims(128, np.array(2), 16, 4, 16) == (None, 16)
     _decode_params(1, np.array(2), 16, 4, 16, 4, torch.float32, torch.float32)
 
 

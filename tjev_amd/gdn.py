@@ -402,6 +402,10 @@ def _check(precision, inverse, chunk, width, key_heads, key_dim, value_heads, va
            conv_weight):
     """gdn_megakernel's checks, in its order and wording (pallas_tpu_mega.py:597-615)."""
     _check_values(precision, inverse, chunk, width, key_heads, key_dim, value_heads, value_dim, heads_per_step)
+    return _conv_taps(conv_weight)
+
+
+def _conv_taps(conv_weight) -> int:
     taps = 1 if conv_weight is None else conv_weight.shape[0]
     if not 1 <= taps <= 5:
         raise ValueError(f"conv kernel of {taps} taps: the megakernel supports 1..5")

@@ -19,7 +19,8 @@ import math
 import torch
 
 from . import _lib
-from .gdn import _check, _plan, _ptr, merge_value_cols, pad_qkv, run_dim, unpad_qkv, value_cols, value_groups
+from .gdn import (_check, _check_values, _conv_taps, _plan, _ptr, merge_value_cols, pad_qkv, run_dim, unpad_qkv,
+                  value_cols, value_groups)
 
 _DTYPES = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16}
 
@@ -103,7 +104,10 @@ def _decode_params(batch, key_heads, key_dim, value_heads, value_dim, taps, io_d
 
 
 @_lib.by_value
-def _decode_dims(key_dim, value_dim):
+def _decode_dims(width, key_heads, key_dim, value_heads, value_dim):
+    """A decode step's head layout, checked, and how its head dims run: their groups of value columns and
+    their padded dim (one lookup for both: each is 0.2 us of the step)."""
+    _check_values("high", "doubling", 64, width, key_heads, key_dim, value_heads, value_dim, 0)
     return value_groups(key_dim, value_dim), run_dim(key_dim, value_dim)
 
 
@@ -116,7 +120,8 @@ def gdn_decode_step(qkv, a, b, a_log, dt_bias, conv_weight, conv_state, state, *
     if qkv.dim() != 2:
         raise ValueError(f"qkv of one token per row is [B, W], not {tuple(qkv.shape)}")
     batch, width = qkv.shape
-    taps = _check("high", "doubling", 64, width, key_heads, key_dim, value_heads, value_dim, 0, conv_weight)
+    groups, run = _decode_dims(width, key_heads, key_dim, value_heads, value_dim)
+    taps = _conv_taps(conv_weight)
     taps = 0 if conv_weight is None else taps
     if not qkv.is_cuda:
         raise RuntimeError("gdn_decode_step runs on the GPU (HIP); got a CPU tensor")
@@ -126,7 +131,6 @@ def gdn_decode_step(qkv, a, b, a_log, dt_bias, conv_weight, conv_state, state, *
         raise ValueError(f"state must be fp32 [{batch}, {value_heads}, {key_dim}, {value_dim}]")
     if taps > 1 and (conv_state is None or conv_state.shape != (batch, taps - 1, width)):
         raise ValueError(f"conv_state must be [{batch}, {taps - 1}, {width}]")
-    groups, run = _decode_dims(key_dim, value_dim)
     if groups is not None:  # value heads wider than 128: groups of value columns (gdn_megakernel's split)
         cut = lambda x, c, w: None if x is None else value_cols(  # noqa: E731
             x, key_heads, key_dim, value_heads, value_dim, c, w)
