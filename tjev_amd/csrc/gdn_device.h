@@ -90,9 +90,9 @@ __device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(ui
 // two values as bf16 (round to nearest even) in one 32-bit word, the first in the low half. As a
 // conversion of a two-element vector it is one v_cvt_pk_bf16_f32; converted one by one and
 // packed it is two of them, a shift and an or (ROCm 7.2). The kernels that stage operands are
-// bound by such instructions beside their loads; measured at the 0.8B layer shape (4 rows of 4096 tokens, 16
-// heads): k_chunk forward 203 -> 191 us, backward 200 -> 188 us, k_out 211 -> 205 us, k_bwd_local 177 ->
-// 172 us, k_bwd_grads (its staging alone) 341 -> 333 us.
+// bound by such instructions beside their loads; measured at the 0.8B layer shape (4 rows of 4096
+// tokens, 16 heads): k_chunk forward 203 -> 191 us, backward 200 -> 188 us, k_out 211 -> 205 us,
+// k_bwd_local 177 -> 172 us, k_bwd_grads (its staging alone) 341 -> 333 us.
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack2(float a, float b) {
@@ -489,7 +489,7 @@ struct Op<P_BF16X3> {
   }
 };
 
-// A 128 x 128 operand as bf16 planes of rows of 16 units of 16 bytes, unit u of row r at u ^ swz(r):
+// An operand of 128 columns as bf16 planes of rows of 16 units of 16 bytes, unit u of row r at u ^ swz(r):
 // 16-byte reads of one unit from 8 consecutive rows and transposing reads of two adjacent units
 // from 4 consecutive rows both fall in distinct banks.
 __device__ __forceinline__ int swz(int r) { return ((r & 3) << 1) | ((r >> 2) & 1); }

@@ -1179,12 +1179,17 @@ struct RawV {
 // ---------------------------------------------------------------- workgroups per CU
 // A chunk kernel's workgroup is one wave per 16 token rows: 4 waves at a chunk of 64, one per
 // SIMD, and its phases (staging, barriers, products) leave the SIMD idle most of the time. At D =
-// 128 in the bf16 modes those kernels keep to half the CU's LDS and registers (operand regions of
-// the operands' own shapes, D x D states staged in two halves) and two workgroups run per CU.
-// Measured at two rows of 1777 tokens, 32 heads (1792 units): k_chunk 89 -> 64 us forward, 107 -> 94
-// backward, k_out 109 -> 79, k_bwd_local 96 -> 66, k_bwd_grads 182 -> 156. (Eight waves per
-// workgroup, two per strip, instead: k_chunk 84 with one workgroup per CU, 83 with two, at 128
-// registers.) At a chunk of 128 the operands alone pass half the LDS.
+// 128 in the bf16 modes those kernels are held to half the CU's LDS (operand regions of the
+// operands' own shapes, D x D states staged in two halves: 57,888 bytes at most) and registers (256),
+// and two workgroups run per CU. Not all of them fit that bound: k_chunk's MODE 1 spills 14-33 VGPRs,
+// k_bwd_grads 6-29, k_out with the norm 1-5 at "high" (none with one workgroup per CU); the first
+// two gain the least. Measured at two rows of 1777 tokens, 32 heads (1792 units): k_chunk 89 -> 64 us
+// forward, 107 -> 94 backward, k_out 109 -> 79, k_bwd_local 96 -> 66, k_bwd_grads 182 -> 156. A grid
+// below the CU count has one workgroup per CU either way and pays for the halves: one row of 300 tokens, 16
+// heads (80 units), k_chunk backward 18.7 -> 20.6 us, k_bwd_grads 26.7 -> 29.1, the whole step's
+// kernels 183 -> 177 us. (Eight waves per workgroup, two per strip, instead: k_chunk 84 us with one
+// workgroup per CU, 83 with two, at 128 registers.) At a chunk of 128 the operands alone pass half
+// the LDS.
 template <int C, int D, int PI>
 constexpr int wgs_per_cu() { return C == 64 && D == 128 && PI != P_F32 ? 2 : 1; }
 
@@ -1243,14 +1248,15 @@ __global__ __launch_bounds__(C * 4, (wgs_per_cu<C, D, PI>())) void k_chunk(GdnAr
   }
   for (int u = blockIdx.x; u < total; u += gridDim.x) {
     const UnitIx<CHUNKS_DOWN> x(A, u);
-    const UnitIx<CHUNKS_DOWN> y(A, u + gridDim.x < total ? u + gridDim.x : u);  // the next unit (or this one again)
+    const UnitIx<CHUNKS_DOWN> y(A, u + gridDim.x < total ? u + gridDim.x : u);  // the next unit (or this one)
     const size_t off = hoff(A, x.b, x.h, A.H, x.n, C, D);
     TinvT<PI>* tg = tinv_ptr<PI>(A) + ((size_t)(x.b * A.H + x.h) * A.N + x.n) * C * C;
     rc.commit(cx);
     if constexpr (!LOAD_T) kk.put_rows(orow);
     rc.fetch(A, y.b, y.h, y.n);
     std::conditional_t<FV, RawV<C, D, NT>, RegsT<C, D, NT>> vc;  // this unit's (v beta)^T source (forward)
-    RegsT<D / NH, D, NT, true, StateT<PS>> sc;  // S_before (one part), its strip of k and its v at the accumulator layout (backward)
+    // S_before (one part), its strip of k and its v at the accumulator layout (backward)
+    RegsT<D / NH, D, NT, true, StateT<PS>> sc;
     StripA<D> ks;
     AccVals<D / 16> va;
     if constexpr (LOAD_T) {
@@ -1826,16 +1832,17 @@ __global__ __launch_bounds__(512) void k_scan_fwd_split(GdnArgs A) {
 // reads of -w's rows, those of P2 (k^T) transposing reads of k's rows (ds_read_b64_tr_b16), so
 // nothing is transposed on its way into LDS (swz_at spreads both kinds of read over the banks).
 // Two barriers per chunk; k and w are loaded a whole chunk step ahead. The order of every
-// accumulation is k_scan_fwd_split's: the same results bit for bit.
+// accumulation is k_scan_fwd_split's (its results were the same bit for bit at C = 128, measured
+// while that form still ran these modes).
 //
-// What bounds it is the CU's memory pipe: 160 KB go through it per step (k and w, 64 KB each, read
-// by every one of a head's four workgroups) with about 56 KB in flight, beside 4 K cycles of LDS
-// per step of about 10 K. Measured against the two-wave form (which transposed k into LDS and left
-// its chunk index in vector registers): one row of 8192 tokens, 32 heads (128 workgroups) 312 -> 281 us; two
-// rows of 2048, 16 heads 76 -> 58 us; 0.8B layer shape (256 workgroups) 185 -> 171 us; chunks of 64
-// against k_scan_fwd (two rows of 1777, 32 heads, segment cuts): 128 -> 90 us. Eight
-// loader waves (168 registers: spills) took 354 us there, w split ahead by k_chunk 292, lines touched three chunks
-// ahead by the compute waves 314.
+// What bounds it is the CU's memory pipe: at C = 128 and fp32 states 176 KB go through it per step
+// (loads: k and w, 64 KB each, read by every one of a head's four workgroups, and 16 KB of u; stores:
+// v_new and S, 16 KB each), beside 4 K cycles of LDS per step of about 10 K. Measured against the
+// two-wave form (which transposed k into LDS and left its chunk index in vector registers): one row of
+// 8192 tokens, 32 heads (128 workgroups) 312 -> 281 us; two rows of 2048, 16 heads 76 -> 58 us; 0.8B
+// layer shape (256 workgroups) 185 -> 171 us; chunks of 64 against k_scan_fwd (two rows of 1777, 32
+// heads, segment cuts): 128 -> 90 us. At one row of 8192 tokens eight loader waves (168 registers: spills) took 354 us, w split ahead by k_chunk 292,
+// lines touched three chunks ahead by the compute waves 314.
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 // the four values of one column (lane % 16) from four rows, 16 columns by four rows per 16 lanes
 // (lane l's address: row (l % 16) / 4, columns 4 (l % 4) .. + 3)
@@ -2178,12 +2185,13 @@ struct RawQ {
 };
 
 // ---------------------------------------------------------------- k_out
-// Persistent: one workgroup per CU (grid <= number of units) loops over the (row, head, chunk)
-// units blockIdx.x, + gridDim.x, ...; C/16 waves. Per unit: o = ((q k^T) . D) v_new + q_read
+// Persistent: wgs_per_cu() workgroups per CU (grid <= number of units) loop over the (row, head,
+// chunk) units blockIdx.x, + gridDim.x, ...; C/16 waves. Per unit: o = ((q k^T) . D) v_new + q_read
 // S_before, token-major output. FQ: q built from the raw rows (RawQ) instead of read from
 // k_prep's rows. Every global input of a unit is held in registers and refilled
 // with the next unit's values right after it has been used, so its loads run during the rest
-// of the unit instead of stalling the next one.
+// of the unit instead of stalling the next one; with states in halves (NH = 2: registers) v_new and
+// S are loaded a stage ahead in their own unit instead.
 template <int C, int D, int NT, class TS, bool FQ = false, int NH = 1>
 struct OutIn {
   CtxRaw<C, FQ> cx;
@@ -2234,7 +2242,6 @@ __global__ __launch_bounds__(C * 4, (wgs_per_cu<C, D, PI>())) void k_out(GdnArgs
     in.cx.commit(cx);
     in.cx.fetch(A, y.b, y.h, y.n);
     in.k.put_rows(orow);
-    // two workgroups per CU: v_new and S come a stage ahead, not a unit ahead (registers)
     if constexpr (NH > 1) in.v.fetch(A.vnew + hoff(A, x.b, x.h, A.H, x.n, C, D), D);
     if constexpr (FQ) in.q.stage(reinterpret_cast<char*>(sI), sWq, A, i0);
     __syncthreads();
@@ -2272,11 +2279,11 @@ __global__ __launch_bounds__(C * 4, (wgs_per_cu<C, D, PI>())) void k_out(GdnArgs
     in.st.put_cols(os);
     // the lane's output row after the quad transposes below (4 consecutive columns per tile)
     const int tok = x.n * C + i0 + ((lane() >> 4) << 2) + (lane() & 3);
-    const size_t orow = (((size_t)x.b * A.T + (tok < A.T ? tok : 0)) * A.H + x.h) * D + (lane() & 12);
+    const size_t ooff = (((size_t)x.b * A.T + (tok < A.T ? tok : 0)) * A.H + x.h) * D + (lane() & 12);
     Raw4<TIO> zr[NORM ? D / 16 : 1];  // the norm's gate, in flight during the last product
     if constexpr (NORM) {
 #pragma unroll
-      for (int t = 0; t < D / 16; ++t) zr[t].load(reinterpret_cast<const TIO*>(A.nz) + orow + 16 * t);
+      for (int t = 0; t < D / 16; ++t) zr[t].load(reinterpret_cast<const TIO*>(A.nz) + ooff + 16 * t);
     }
     if constexpr (NH == 1) {
       __syncthreads();
@@ -2301,7 +2308,7 @@ __global__ __launch_bounds__(C * 4, (wgs_per_cu<C, D, PI>())) void k_out(GdnArgs
       for (int t = 0; t < D / 16; ++t) {
         float v[4] = {o[t][0], o[t][1], o[t][2], o[t][3]};
         quad_transpose(v);
-        if (tok < A.T) st4_io(out + orow + 16 * t, v);
+        if (tok < A.T) st4_io(out + ooff + 16 * t, v);
         if constexpr (NORM) {  // the norm reads out as stored
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
@@ -2324,7 +2331,7 @@ __global__ __launch_bounds__(C * 4, (wgs_per_cu<C, D, PI>())) void k_out(GdnArgs
 #pragma unroll
           for (int e = 0; e < 4; ++e)
             yv[e] = valid ? wv[e] * rnd_io<TIO>(o[t][e] * r) * (z[e] * sigmoid_io<TIO>(z[e])) : 0.f;
-          if (tok < A.T) st4_io(reinterpret_cast<TIO*>(A.ny) + orow + 16 * t, yv);
+          if (tok < A.T) st4_io(reinterpret_cast<TIO*>(A.ny) + ooff + 16 * t, yv);
         }
       }
     }
@@ -2334,7 +2341,7 @@ __global__ __launch_bounds__(C * 4, (wgs_per_cu<C, D, PI>())) void k_out(GdnArgs
 
 // ---------------------------------------------------------------- k_tail
 // The decode state a prefill leaves, in one launch of 256-thread workgroups: the recurrent state
-// after token T-1 of each row (the first tail_blocks() workgroups, when final_state is given) and
+// after token T-1 of each row (the first B H PER_HEAD workgroups, when final_state is given) and
 // the conv history (the rest, when conv_state is given).
 //
 // The recurrent state (xla.py:141-167 run to the last token) is the scan's update of the last
@@ -2359,8 +2366,8 @@ struct TailTile {
 template <int C, int D, class TIO>
 __global__ __launch_bounds__(256) void k_tail(GdnArgs A) {
   constexpr int R = TailTile<D>::R, T = TailTile<D>::T;
-  // row strides of 16 words modulo the 64 banks: the four token rows that one MFMA operand read
-  // spans fall in distinct banks
+  // row strides of 16 or 48 words modulo the 64 banks: the four token rows that one MFMA operand
+  // read spans fall in distinct banks (at D = 16 of 32 words: two rows share theirs)
   constexpr int LK = R + 16, LV = T + 16;
   __shared__ __align__(16) float sk[C * LK];
   __shared__ __align__(16) float sv[C * LV];
